@@ -11,13 +11,13 @@
 // Decomposition.  A workgroup of WAVES waves owns WAVES * NW 16-column tiles of the output
 // and a K range of `kt` elements; gridDim.y workgroups split K, and when it exceeds one they
 // write fp32 partials that reduce_kernel sums in a fixed order (deterministic, no atomics).
-//   * W streams from HBM straight into MFMA B operands: per 128-wide K step a lane reads 64
+//   * W streams from HBM straight into MFMA A operands: per 128-wide K step a lane reads 64
 //     contiguous bytes of its output row as 4 x 16 B (MFMA j covers k0 + 32j + [8g, 8g+8),
 //     g = lane / 16), PF steps ahead of the MFMAs.
 //   * X is shared: each K step's [M, 128] slice is staged once per workgroup in LDS (double
-//     buffered, rows padded to 272 bytes) and read by all waves as MFMA A operands.
-//   * v_mfma_f32_16x16x32_bf16 with A = X rows, B = W rows: lane l holds
-//     C[4(l/16) + i][l % 16] of each 16x16 tile.
+//     buffered, rows padded to 288 bytes) and read by all waves as MFMA B operands.
+//   * v_mfma_f32_16x16x32_bf16 with A = W rows, B = X rows: lane l holds
+//     C^T[4(l/16) + i][l % 16] of each 16x16 tile, four consecutive columns of one row.
 //
 // Tile-packed weights (coopt_linear_pack_weight).  W may instead be stored as [N/16][K/128]
 // tiles of 16 rows x 128 K, each the 4 x 64 16-byte chunks in the order the lanes load them:
@@ -34,7 +34,12 @@ typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 
 constexpr int kKB = 128;                  // K elements per step
-constexpr int kPitch = kKB * 2 + 16;      // LDS bytes per staged X row
+// LDS bytes per staged X row.  A fragment read has 16 lanes at consecutive rows and four 16-byte
+// columns; at a pitch of 288 it takes 4.1 cycles per 1 KB, the rate of a contiguous read, at 272
+// (one 16-byte unit of padding) 7.0: bank conflicts on 41 of the 93 kcycles the LDS was busy in
+// a 160 x 28672 x 4096 call.  160 rows, partials: gate_up 64 -> 57 us, down 35.1 -> 31.9, qkv
+// 24.6 -> 23.0.
+constexpr int kPitch = kKB * 2 + 32;
 
 struct LinArgs {
   const uint16_t* x;
@@ -58,19 +63,22 @@ __device__ __forceinline__ f32x4_t mfma_bf16(u32x4_t a, u32x4_t b, f32x4_t c) {
                                                  __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
 }
 
+template <bool NT = false>
 __device__ __forceinline__ u32x4_t ldg16(const uint16_t* p) {
-  return *reinterpret_cast<const u32x4_t*>(p);
+  const u32x4_t* q = reinterpret_cast<const u32x4_t*>(p);
+  return NT ? __builtin_nontemporal_load(q) : *q;
 }
 
 // MT: 16-row tiles of M; NW: 16-column tiles per wave; WAVES: waves per workgroup;
-// PF: K steps of W in flight per wave (even); PK: W is tile-packed; SILU: W is a gate_up
+// PF: K steps of W in flight per wave (even); PK: W is tile-packed; NT: W is loaded with the
+// nontemporal hint (nt_for); SILU: W is a gate_up
 // weight packed with gate and up tiles interleaved (coopt_linear_pack_gate_up), K is not
 // split, and the output is silu(gate) * up (F = N / 2 columns) instead of the projection.
 // The arguments are scalars, not a LinArgs by value: the first sixteen kernel-argument dwords
 // (x through ldy) are then preloaded into SGPRs (the build's kernarg-preload option), so the
 // first X / W loads do not wait for a kernel-argument load; part and force_part, needed only
 // at the end, load from the segment.
-template <int MT, int NW, int WAVES, int PF, bool PK, bool SILU = false>
+template <int MT, int NW, int WAVES, int PF, bool PK, bool NT, bool SILU = false>
 __global__ __launch_bounds__(64 * WAVES) void linear_kernel(
     const uint16_t* x, int64_t ldx, const uint16_t* w, int64_t ldw, int M, int N, int K, int kt,
     uint16_t* y, int64_t ldy, float* part, int force_part) {
@@ -80,7 +88,9 @@ __global__ __launch_bounds__(64 * WAVES) void linear_kernel(
   constexpr int kThreads = 64 * WAVES;
   constexpr int kRowsPerRound = kThreads / 16;                     // X rows staged per round
   constexpr int kRounds = (MT * 16 + kRowsPerRound - 1) / kRowsPerRound;
-  __shared__ __attribute__((aligned(16))) unsigned char xs[2][MT * 16 * kPitch];
+  // whole rounds are staged: with a row count that the rounds do not divide, the rows past it
+  // get LDS of their own rather than a branch around the store
+  __shared__ __attribute__((aligned(16))) unsigned char xs[2][kRounds * kRowsPerRound * kPitch];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int l16 = lane & 15, g = lane >> 4;
   const int n0 = (blockIdx.x * WAVES + wave) * NW * 16;
@@ -107,16 +117,14 @@ __global__ __launch_bounds__(64 * WAVES) void linear_kernel(
     }
   }
   // X staging: in round r, thread t loads 16 B of row r * kRowsPerRound + t / 16 at byte
-  // 16 (t % 16) of the step; rows >= 16 MT are not staged.  Rows in [M, 16 MT) repeat row
+  // 16 (t % 16) of the step.  Rows past M repeat row
   // M - 1: their outputs are never stored, and an unconditional load keeps the compiler's
   // load counting exact (a load under a branch makes it wait for every load in flight).
   const int xr_row = threadIdx.x >> 4, xr_col = (threadIdx.x & 15) * 8;
   const uint16_t* xrow[kRounds];
-  bool xin[kRounds];
 #pragma unroll
   for (int r = 0; r < kRounds; ++r) {
     const int m = r * kRowsPerRound + xr_row;
-    xin[r] = m < MT * 16;
     xrow[r] = a.x + static_cast<int64_t>(m < a.M ? m : a.M - 1) * a.ldx + kbeg + xr_col;
   }
 
@@ -128,14 +136,12 @@ __global__ __launch_bounds__(64 * WAVES) void linear_kernel(
 #pragma unroll
     for (int nt = 0; nt < NW; ++nt)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) wr[nt][j] = ldg16(wrow[nt] + s * kWStep + kWChunk * j);
+      for (int j = 0; j < 4; ++j) wr[nt][j] = ldg16<NT>(wrow[nt] + s * kWStep + kWChunk * j);
   };
   auto store_x = [&](int buf, const u32x4_t (&xr)[kRounds]) {
 #pragma unroll
     for (int r = 0; r < kRounds; ++r)
-      if (xin[r])
-        *reinterpret_cast<u32x4_t*>(
-            &xs[buf][(r * kRowsPerRound + xr_row) * kPitch + xr_col * 2]) = xr[r];
+      *reinterpret_cast<u32x4_t*>(&xs[buf][(r * kRowsPerRound + xr_row) * kPitch + xr_col * 2]) = xr[r];
   };
 
   f32x4_t acc[MT][NW];
@@ -156,7 +162,7 @@ __global__ __launch_bounds__(64 * WAVES) void linear_kernel(
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-      for (int nt = 0; nt < NW; ++nt) acc[mt][nt] = mfma_bf16(fa[mt], wr[nt][j], acc[mt][nt]);
+      for (int nt = 0; nt < NW; ++nt) acc[mt][nt] = mfma_bf16(wr[nt][j], fa[mt], acc[mt][nt]);
   };
   // (sched_barrier keeps the scheduler from sinking the reads back next to their MFMAs)
   auto compute = [&](int buf, const u32x4_t (&wr)[NW][4]) {
@@ -202,62 +208,73 @@ __global__ __launch_bounds__(64 * WAVES) void linear_kernel(
     }
   }
 
-  // Epilogue: lane holds rows 16 mt + 4 g + i of column n0 + 16 nt + l16.
+  // Epilogue.  W is the MFMAs' A operand and X their B, so a lane holds four consecutive
+  // columns, n0 + 16 nt + 4 g + i, of row 16 mt + l16: one 16-byte (bf16: 8-byte) store per tile
+  // instead of four of one column each.
+  auto pack4 = [](const f32x4_t& v) {
+    return make_uint2(f32_to_bf16(v[0]) | (static_cast<uint32_t>(f32_to_bf16(v[1])) << 16),
+                      f32_to_bf16(v[2]) | (static_cast<uint32_t>(f32_to_bf16(v[3])) << 16));
+  };
   if constexpr (SILU) {
     // Wave 2p holds gate tile t = blockIdx.x * WAVES / 2 + p and wave 2p + 1 the matching up
-    // tile; the up wave hands its sums over through LDS (the X staging is dead by now).  Each
-    // sum is rounded to bf16 first -- the projection's output -- then silu(gate) * up as
-    // silu_mul_kernel computes it, rounded once more.
+    // tile.  They hand each other half of their row tiles through LDS (the X staging is dead by
+    // now) and finish the other half each.  Each sum is rounded to bf16 first -- the
+    // projection's output -- then silu(gate) * up as silu_mul_kernel computes it, rounded once
+    // more.  (With the up waves handing over everything and ending there, 160 x 28672 x 4096 took
+    // 3 us more.)
+    constexpr int kHalf = (MT + 1) / 2;  // row tiles the gate wave finishes
     __syncthreads();
-    float* xch = reinterpret_cast<float*>(&xs[0][0]);
-    const int pair = wave >> 1;
-    if (wave & 1) {
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) xch[((pair * MT + mt) * 4 + i) * 64 + lane] = acc[mt][0][i];
-    }
-    __syncthreads();
-    if (wave & 1) return;
+    f32x4_t* xch = reinterpret_cast<f32x4_t*>(&xs[0][0]) + (wave >> 1) * (MT * 64) + lane;
     const int F = a.N / 2;
-    const int j = (blockIdx.x * (WAVES / 2) + pair) * 16 + l16;
-    if (j >= F) return;
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
+    const int j = (blockIdx.x * (WAVES / 2) + (wave >> 1)) * 16 + 4 * g;
+    auto finish = [&](int mt, const f32x4_t& gate, const f32x4_t& up) {
+      const int m = mt * 16 + l16;
+      f32x4_t r;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const int m = mt * 16 + 4 * g + i;
-        if (m >= a.M) continue;
-        const float gv = bf16_to_f32(f32_to_bf16(acc[mt][0][i]));
-        const float uv = bf16_to_f32(f32_to_bf16(xch[((pair * MT + mt) * 4 + i) * 64 + lane]));
-        a.y[static_cast<int64_t>(m) * a.ldy + j] = f32_to_bf16(gv / (1.0f + __expf(-gv)) * uv);
+        const float gv = bf16_to_f32(f32_to_bf16(gate[i]));
+        const float uv = bf16_to_f32(f32_to_bf16(up[i]));
+        r[i] = gv / (1.0f + __expf(-gv)) * uv;
       }
+      if (m < a.M && j < F)
+        *reinterpret_cast<uint2*>(a.y + static_cast<int64_t>(m) * a.ldy + j) = pack4(r);
+    };
+    if (wave & 1) {
+#pragma unroll
+      for (int mt = 0; mt < kHalf; ++mt) xch[mt * 64] = acc[mt][0];
+      __syncthreads();
+#pragma unroll
+      for (int mt = kHalf; mt < MT; ++mt) finish(mt, xch[mt * 64], acc[mt][0]);
+    } else {
+#pragma unroll
+      for (int mt = kHalf; mt < MT; ++mt) xch[mt * 64] = acc[mt][0];
+      __syncthreads();
+#pragma unroll
+      for (int mt = 0; mt < kHalf; ++mt) finish(mt, acc[mt][0], xch[mt * 64]);
+    }
     return;
   }
   if (gridDim.y == 1 && !a.force_part) {
 #pragma unroll
     for (int nt = 0; nt < NW; ++nt) {
-      const int n = n0 + nt * 16 + l16;
+      const int n = n0 + nt * 16 + 4 * g;
       if (n >= a.N) continue;
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int m = mt * 16 + 4 * g + i;
-          if (m < a.M) a.y[static_cast<int64_t>(m) * a.ldy + n] = f32_to_bf16(acc[mt][nt][i]);
-        }
+      for (int mt = 0; mt < MT; ++mt) {
+        const int m = mt * 16 + l16;
+        if (m < a.M)
+          *reinterpret_cast<uint2*>(a.y + static_cast<int64_t>(m) * a.ldy + n) = pack4(acc[mt][nt]);
+      }
     }
   } else {
     float* p = a.part + static_cast<int64_t>(blockIdx.y) * (MT * 16) * a.N;
 #pragma unroll
     for (int nt = 0; nt < NW; ++nt) {
-      const int n = n0 + nt * 16 + l16;
+      const int n = n0 + nt * 16 + 4 * g;
       if (n >= a.N) continue;
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          p[static_cast<int64_t>(mt * 16 + 4 * g + i) * a.N + n] = acc[mt][nt][i];
+        *reinterpret_cast<f32x4_t*>(p + static_cast<int64_t>(mt * 16 + l16) * a.N + n) = acc[mt][nt];
     }
   }
 }
@@ -336,14 +353,25 @@ Plan plan_for(int M, int N, int K) {
   return p;
 }
 
+// Packed weights are loaded with the nontemporal hint where a slice has at least 16 K steps:
+// 160 x 28672 x 4096 55.5 -> 53 us, 32 x 16384 x 2048 15.5 -> 14.1, 16 x 4096 x 14336 (4 slices of
+// 28 steps) 22.8 -> 20.7.  Shorter slices keep plain loads: the reload of a slice's last step (the
+// pipeline's clamped tail) then hits the L2, and the partials' reader found more of them
+// cached (160 x 6144 x 4096 with its reduction 24.5 us plain, 26.3 with the hint).  Row-major
+// weights keep them too (a load covers half of each of 16 rows' lines: 66 -> 72 us).
+bool nt_for(const Plan& p) { return p.kt >= 16 * kKB; }
+
 template <int MT, int NW, int WAVES, int PF>
 void launch_cfg(const Plan& p, const LinArgs& a, bool packed, hipStream_t s) {
   const int cols = WAVES * NW * 16;
   const dim3 grid((a.N + cols - 1) / cols, p.ks);
-  if (packed)
-    hipLaunchKernelGGL((linear_kernel<MT, NW, WAVES, PF, true>), grid, dim3(64 * WAVES), 0, s, LIN_ARGS(a));
+  const dim3 block(64 * WAVES);
+  if (!packed)
+    hipLaunchKernelGGL((linear_kernel<MT, NW, WAVES, PF, false, false>), grid, block, 0, s, LIN_ARGS(a));
+  else if (nt_for(p))
+    hipLaunchKernelGGL((linear_kernel<MT, NW, WAVES, PF, true, true>), grid, block, 0, s, LIN_ARGS(a));
   else
-    hipLaunchKernelGGL((linear_kernel<MT, NW, WAVES, PF, false>), grid, dim3(64 * WAVES), 0, s, LIN_ARGS(a));
+    hipLaunchKernelGGL((linear_kernel<MT, NW, WAVES, PF, true, false>), grid, block, 0, s, LIN_ARGS(a));
 }
 
 template <int MT>
@@ -463,12 +491,15 @@ int pack_weight(const void* w, int64_t ldw, int N, int K, int gu_half, void* out
 }
 
 template <int MT, int WAVES>
-void launch_silu(int F, const LinArgs& a, hipStream_t s) {
+void launch_silu(const Plan& p, int F, const LinArgs& a, hipStream_t s) {
   // WAVES / 2 (gate, up) tile pairs per workgroup; pairs of a trailing partial workgroup past
   // the weight read clamped tiles and write nothing (their columns are >= F)
   const int rows = 16 * WAVES;
-  hipLaunchKernelGGL((linear_kernel<MT, 1, WAVES, 2, true, true>), dim3((2 * F + rows - 1) / rows, 1),
-                     dim3(64 * WAVES), 0, s, LIN_ARGS(a));
+  const dim3 grid((2 * F + rows - 1) / rows, 1), block(64 * WAVES);
+  if (nt_for(p))
+    hipLaunchKernelGGL((linear_kernel<MT, 1, WAVES, 2, true, true, true>), grid, block, 0, s, LIN_ARGS(a));
+  else
+    hipLaunchKernelGGL((linear_kernel<MT, 1, WAVES, 2, true, false, true>), grid, block, 0, s, LIN_ARGS(a));
 }
 
 }  // namespace
@@ -512,10 +543,10 @@ extern "C" int coopt_linear_silu_packed(const void* x, int64_t ldx, const void* 
             2 * F, K, p.kt, static_cast<uint16_t*>(y), ldy, nullptr, 0};
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   switch (p.mt) {
-    case 1: launch_silu<1, 4>(F, a, s); break;
-    case 2: launch_silu<2, 4>(F, a, s); break;
-    case 4: launch_silu<4, 4>(F, a, s); break;
-    default: launch_silu<10, 8>(F, a, s); break;   // the verify rows (129-160), 8 waves
+    case 1: launch_silu<1, 4>(p, F, a, s); break;
+    case 2: launch_silu<2, 4>(p, F, a, s); break;
+    case 4: launch_silu<4, 4>(p, F, a, s); break;
+    default: launch_silu<10, 8>(p, F, a, s); break;   // the verify rows (129-160), 8 waves
   }
   return coopt::check_launch("coopt_linear_silu_packed");
 }

@@ -102,12 +102,12 @@ class RandomLlama:
         self.scale = 1.0 / math.sqrt(D)
 
     # Projections kept tile-packed as well on the GPU: those that stream through coopt_linear
-    # at verify row counts.  A model run only at draft row counts (<= 64) streams gate_up
-    # through it too, and its logits projection, and passes
+    # at verify row counts, gate_up with its SiLU fused (160 rows of the 8B widths: 54 us against
+    # 57 + 6 us of torch's GEMM and silu_and_mul).  A model run only at draft row counts (<= 64)
+    # streams its logits projection through it too, and passes
     # packed=("qkv", "o", "gate_up", "down", "lm_head").  At 160 rows the target's lm_head
-    # runs on torch's GEMM, and so does its gate_up: the fused gate_up + SiLU kernel takes 160
-    # rows too, but the step measured 11.72 ms with it against 11.58 ms with hipBLASLt.
-    PACKED = ("qkv", "o", "down")
+    # runs on torch's GEMM (245 us; coopt_linear_packed 242).
+    PACKED = ("qkv", "o", "gate_up", "down")
 
     def _pack(self):
         ok = lambda w, r=16: w.shape[0] % r == 0 and w.shape[1] % 128 == 0  # tile granularity
