@@ -11,7 +11,7 @@
 // the block's start-up round trips overlap.  The waves merge through LDS, each into its own
 // region in one round, summed while the output is written.  With one split the block writes
 // the bf16 output; otherwise it writes its (max, sum) and unnormalised fp32 rows to the
-// workspace and a second launch (merge_kernel, one block per (KV head, sequence)) combines
+// workspace and a second launch (merge_kernel, one wave per row) combines
 // the splits -- the kernel boundary orders the two, so no block waits on another and no
 // cross-workgroup fence is needed.  A ragged batch with more (sequence, KV head) items than
 // one round of blocks holds runs on a 1-D grid whose blocks rank the sequences by length and
@@ -304,8 +304,9 @@ __global__ __launch_bounds__(64 * waves_for(RT), 1) void verify_attn_kernel(
   typedef const __attribute__((address_space(4))) int32_t* const_i32_ptr;
   const int64_t bt_last = bt_stride - 1;
   // The pages of the wave's first tile of piece sidx of sequence b, looked up before L is
-  // known: they are used only if that tile is full, i.e. all its keys are < L, where no
-  // clamp to L - 1 applies (the index is kept inside the table row regardless).
+  // known, so not clamped to the last key's page: a half tile past the end may get whatever
+  // page its table entry names, clamped into the pool, and clear_tail drops what is read there
+  // (the index is kept inside the table row regardless).
   auto first_pages = [&](int b, int sidx, int32_t& p0, int32_t& p1) {
     const const_i32_ptr tb = (const_i32_ptr)(bt_p + static_cast<int64_t>(b) * bt_stride);
     const int kb = sidx * split + wave * kTileKeys;
@@ -484,9 +485,7 @@ __global__ __launch_bounds__(64 * waves_for(RT), 1) void verify_attn_kernel(
   };
 
   // Issue every load of tile `t` (pages pg0/pg1).  Page bases are wave-uniform (scalar);
-  // lanes add 32-bit byte offsets.  Full tiles (every key < L) use offsets fixed for the
-  // whole loop; the last, partial tile clamps each key to L - 1, so no row past the
-  // sequence is read.
+  // lanes add 32-bit byte offsets, fixed for the whole loop.
   const int c_ts = static_cast<int>(a.c_ts), s_ts = static_cast<int>(a.s_ts);
   const uint32_t k_lane = kElt * l16 * c_ts + 16 * grp;
   uint32_t v_lane[4];
@@ -509,10 +508,9 @@ __global__ __launch_bounds__(64 * waves_for(RT), 1) void verify_attn_kernel(
       load_words<Raw::kVWords>(vp + off, raw.v[kt * 4 + i]);
     }
   };
-  // a full tile: every key < L
   // INT8: the scales are issued first, so the V-scale check of a loaded tile (vcheck) waits
   // only for them and leaves the tile's K/V loads in flight.
-  auto load_full = [&](Raw& raw, int t, int64_t pg0, int64_t pg1) {
+  auto load_tile = [&](Raw& raw, int t, int64_t pg0, int64_t pg1) {
     const int kb = k_begin + t * kTileKeys;
     if constexpr (INT8) {
 #pragma unroll
@@ -543,32 +541,21 @@ __global__ __launch_bounds__(64 * waves_for(RT), 1) void verify_attn_kernel(
       issue(raw, kt, kbase + kElt * r, vbase + kElt * r, k_lane, v_lane);
     }
   };
-  // the split's last tile when it ends inside a tile: keys clamped to L - 1
-  auto load_partial = [&](Raw& raw, int t, int64_t pg0, int64_t pg1) {
-    const int kb = k_begin + t * kTileKeys;
+  // The split's last tile when the sequence ends inside it: loaded like the others (the rows
+  // past the end lie in the same page, or in some page of the pool), then the values of the
+  // keys past the end are zeroed -- their probabilities are 0, but 0 times whatever a row that
+  // was never written holds need not be -- and with them the V scales vcheck looks at.
+  auto clear_tail = [&](Raw& raw, int t) {
+    // keys of the tile inside the split, from the lane's first one on (the asm keeps eight
+    // comparands from being held in registers through the loop)
+    int left = k_end - (k_begin + t * kTileKeys) - grp * 4;
+    asm volatile("" : "+v"(left));
 #pragma unroll
-    for (int kt = 0; kt < 2; ++kt) {
-      const int64_t pg = kt ? pg1 : pg0;
-      const int sub = kb + kt * 16;
-      const int64_t row0 = pg * a.c_bs + head_off;
-      const int ktk = min(sub + l16, L - 1) & bs_mask;
-      const uint32_t ko = kElt * ktk * c_ts + 16 * grp;
-      uint32_t vo[4], tk[4];
+    for (int j = 0; j < 8; ++j) {
+      const uint32_t keep = (j >> 2) * 16 + (j & 3) < left ? 0xffffffffu : 0u;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        tk[i] = min(sub + grp * 4 + i, L - 1) & bs_mask;
-        vo[i] = kElt * (tk[i] * c_ts + l16 * kDt);
-      }
-      issue(raw, kt, kbase + kElt * row0, vbase + kElt * row0, ko, vo);
-      if constexpr (INT8) {
-        const uint16_t* ksp = a.ks + pg * a.s_bs + shead_off;
-        const uint16_t* vsp = a.vs + pg * a.s_bs + shead_off;
-        raw.ks[kt] = ksp[ktk * s_ts];
-        uint32_t vh[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) vh[i] = vsp[tk[i] * s_ts];
-        raw.vs[kt] = u32x2_t{vh[0] | (vh[1] << 16), vh[2] | (vh[3] << 16)};
-      }
+      for (int w = 0; w < Raw::kVWords; ++w) raw.v[j][w] &= keep;
+      if constexpr (INT8) raw.vs[j >> 2][(j >> 1) & 1] &= (j & 1) ? (keep | 0xffffu) : (keep | 0xffff0000u);
     }
   };
 
@@ -779,83 +766,65 @@ __global__ __launch_bounds__(64 * waves_for(RT), 1) void verify_attn_kernel(
   };
 
   // ---- the wave's tiles: double-buffered (the next tile's loads in flight while the current
-  // one is computed) or, for large row counts, one at a time; then the partial tile ----
+  // one is computed) or, for large row counts, one at a time ----
   // Wave w takes tiles w, w + kWaves, w + 2 kWaves, ... (a fixed assignment keeps the result
-  // bit-reproducible: each wave's sum covers the same keys on every call); the wave whose
-  // sequence reaches nfull also takes the split's partial tile.
-  const int nfull = (k_end - k_begin) / kTileKeys;
+  // bit-reproducible: each wave's sum covers the same keys on every call).  The split's partial
+  // last tile is one of them: loaded behind the full ones with a load of its own after the
+  // loop, it cost its wave a memory round trip (1 sequence, 717 keys, unsplit: 11.6 us, 11.3 in the loop).
   auto pages = [&](int t, int64_t& p0, int64_t& p1) {
     const int kb = k_begin + t * kTileKeys;
     p0 = page_of(kb);
     p1 = page_of(kb + 16);
   };
-  bool own_partial = wave == nfull;
-  int next_t = wave + kWaves;
-  auto grab = [&]() {
-    const int v = next_t;
-    next_t += kWaves;
-    own_partial |= v == nfull;
-    return v;
+  // a loaded tile, before it is computed
+  auto prepare = [&](Raw& raw, int t) {
+    if (k_begin + (t + 1) * kTileKeys > k_end) clear_tail(raw, t);
+    vcheck(raw);
   };
   if constexpr (DB) {
-    // Loads inside the loop are unconditional (an index past the last full tile repeats it,
+    // Loads inside the loop are unconditional (an index past the last tile repeats it,
     // already cached, and is never computed), so each compute waits only for its own
     // buffer's loads and the other buffer's stay in flight.
     Raw bufA, bufB;
-    const int tlast = nfull - 1;
+    const int tlast = ntiles - 1;
     int tA = wave;
     int64_t nx0 = 0, nx1 = 0;  // pages of the wave's next tile to load
     // fused: a first tile holding keys this launch writes ([L - n, L)) loads after the barrier
     const bool defer = fused && k_begin + (tA + 1) * kTileKeys > L - n;
-    if (tA < nfull && !defer) load_full(bufA, tA, first_pg0, first_pg1);
+    if (tA < ntiles && !defer) load_tile(bufA, tA, first_pg0, first_pg1);
     stage_q();  // the Q loads complete while the first tile's are in flight
-    if (tA < nfull && defer) load_full(bufA, tA, first_pg0, first_pg1);
-    if (tA < nfull) {
-      vcheck(bufA);
-      int tB = grab();
+    if (tA < ntiles && defer) load_tile(bufA, tA, first_pg0, first_pg1);
+    if (tA < ntiles) {
+      prepare(bufA, tA);
+      int tB = tA + kWaves;
       pages(min(tB, tlast), nx0, nx1);
       for (;;) {
-        load_full(bufB, min(tB, tlast), nx0, nx1);
-        const int tA2 = tB < nfull ? grab() : nfull;
+        load_tile(bufB, min(tB, tlast), nx0, nx1);
+        const int tA2 = tB + kWaves;
         pages(min(tA2, tlast), nx0, nx1);
         compute_tile(bufA, tA);
-        vcheck(bufB);
-        if (tB >= nfull) break;
-        load_full(bufA, min(tA2, tlast), nx0, nx1);
-        const int tB2 = tA2 < nfull ? grab() : nfull;
+        if (tB >= ntiles) break;
+        prepare(bufB, tB);
+        load_tile(bufA, min(tA2, tlast), nx0, nx1);
+        const int tB2 = tA2 + kWaves;
         pages(min(tB2, tlast), nx0, nx1);
         compute_tile(bufB, tB);
-        vcheck(bufA);
-        if (tA2 >= nfull) break;
+        if (tA2 >= ntiles) break;
+        prepare(bufA, tA2);
         tA = tA2;
         tB = tB2;
       }
     }
   } else {
     Raw buf;
-    int64_t nx0 = 0, nx1 = 0;
-    int t = wave;
-    if (t < nfull) {
-      nx0 = first_pg0;
-      nx1 = first_pg1;
-    }
+    int64_t nx0 = first_pg0, nx1 = first_pg1;
     stage_q();
-    while (t < nfull) {
-      load_full(buf, t, nx0, nx1);
-      const int tn = grab();
-      if (tn < nfull) pages(tn, nx0, nx1);
-      vcheck(buf);
+    for (int t = wave; t < ntiles; t += kWaves) {
+      load_tile(buf, t, nx0, nx1);
+      if (t + kWaves < ntiles) pages(t + kWaves, nx0, nx1);
+      prepare(buf, t);
       compute_tile(buf, t);
-      t = tn;
     }
-  }
-  if (nfull < ntiles && own_partial) {
-    Raw buf;
-    int64_t p0, p1;
-    pages(nfull, p0, p1);
-    load_partial(buf, nfull, p0, p1);
-    vcheck(buf);
-    compute_tile(buf, nfull);
   }
   // ---- merge the waves ----
   // the wave's o and l are relative to 2^(m_run + e_v) (e_v = 0 for bf16 KV)
@@ -1055,48 +1024,90 @@ __global__ __launch_bounds__(64 * waves_for(RT), 1) void verify_attn_kernel(
 // than one split.  Stream order makes the first launch's stores visible here; no fences or
 // counters are involved (an agent-scope fence per block writes back and invalidates the L2
 // of this multi-XCD part and costs far more than the extra launch).
+// Latency bounds it (a few MB at most), so one wave takes one row: D / 8 lanes cover the row, the
+// rest of the wave the splits, kSG at a time with two rounds' loads in flight, and the split
+// groups' sums meet in lane exchanges.  4 sequences x 8 KV heads x 20 rows of 5 to 8 splits: 12.1
+// us with one block per (sequence, KV head) walking the splits in turn, 3.5 like this.
 template <int D>
 __global__ __launch_bounds__(kThreads) void merge_kernel(AttnArgs a) {
-  const int b = blockIdx.y, hkv = blockIdx.x;
+  constexpr int kCh = D / 8;         // lanes per row
+  constexpr int kSG = 64 / kCh;      // splits per round
+  constexpr int kUnroll = 2;         // rounds whose loads are issued together
+  const int b = blockIdx.y, lane = threadIdx.x & 63;
+  const int item = blockIdx.x * (kThreads / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int hkv = item / a.rmax, r = item - hkv * a.rmax;
   const int q0 = a.cu[b];
   const int n = a.cu[b + 1] - q0;
   const int L = min(a.seq_lens[b], a.max_seqlen_k);
-  if (n <= 0) return;
+  if (hkv >= a.Hkv || n <= 0 || r >= a.G * n) return;
   const int nsplit = L > 0 ? (L + a.split - 1) / a.split : 1;
   if (nsplit <= 1) return;
-  const int R = min(a.G * n, a.rmax);
-  constexpr int kCh = D / 8;
-  const int64_t first = (static_cast<int64_t>(b) * a.Hkv + hkv) * a.max_splits;
-  auto slot = [&](int s) { return (first + s) * a.rmax; };
-  for (int idx = threadIdx.x; idx < R * kCh; idx += kThreads) {
-    const int r = idx / kCh, c = idx % kCh;
-    float M = -INFINITY;
-    for (int s = 0; s < nsplit; ++s) M = fmaxf(M, a.part_ml[slot(s) + r].x);
-    f32x4_t acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f};
-    float Lsum = 0.0f;
-    for (int s = 0; s < nsplit; ++s) {
-      const float2 ml = a.part_ml[slot(s) + r];
-      if (!(ml.x > -INFINITY)) continue;
-      const float w = exp2_fast(ml.x - M);
-      Lsum += ml.y * w;
-      const f32x4_t* src = reinterpret_cast<const f32x4_t*>(a.part_o + (slot(s) + r) * D + c * 8);
-      acc0 += src[0] * w;
-      acc1 += src[1] * w;
+  const int c = lane % kCh, sg = lane / kCh;
+  const int64_t row0 = (static_cast<int64_t>(b) * a.Hkv + hkv) * a.max_splits * a.rmax + r;
+  float M = -INFINITY, Lsum = 0.0f;
+  f32x4_t acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f};
+  for (int s0 = 0; s0 < nsplit; s0 += kSG * kUnroll) {
+    float2 ml[kUnroll];
+    f32x4_t x0[kUnroll], x1[kUnroll];
+#pragma unroll
+    for (int u = 0; u < kUnroll; ++u) {
+      const int s = s0 + u * kSG + sg;  // past the last split: its row again, with weight 0
+      const int64_t row = row0 + static_cast<int64_t>(min(s, nsplit - 1)) * a.rmax;
+      ml[u] = a.part_ml[row];
+      const f32x4_t* src = reinterpret_cast<const f32x4_t*>(a.part_o + row * D + c * 8);
+      x0[u] = src[0];
+      x1[u] = src[1];
     }
-    const float inv = Lsum > 0.0f ? 1.0f / Lsum : 0.0f;
-    const u32x4_t v = {pack_bf16x2(acc0[0] * inv, acc0[1] * inv), pack_bf16x2(acc0[2] * inv, acc0[3] * inv),
-                       pack_bf16x2(acc1[0] * inv, acc1[1] * inv), pack_bf16x2(acc1[2] * inv, acc1[3] * inv)};
-    const int hl = r / n, j = r - hl * n;
-    uint16_t* dst = a.out + static_cast<int64_t>(q0 + j) * a.o_ts +
-                    static_cast<int64_t>(hkv * a.G + hl) * a.o_hs + c * 8;
-    *reinterpret_cast<u32x4_t*>(dst) = v;
+    float m_new = M;
+#pragma unroll
+    for (int u = 0; u < kUnroll; ++u) {
+      if (s0 + u * kSG + sg >= nsplit) ml[u].x = -INFINITY;
+      m_new = fmaxf(m_new, ml[u].x);
+    }
+    const float f = M > -INFINITY ? exp2_fast(M - m_new) : 0.0f;
+    Lsum *= f;
+    acc0 *= f;
+    acc1 *= f;
+#pragma unroll
+    for (int u = 0; u < kUnroll; ++u) {
+      // a split without a visible key has no sums worth reading (its maximum is -inf)
+      if (!(ml[u].x > -INFINITY)) continue;
+      const float w = exp2_fast(ml[u].x - m_new);
+      Lsum += ml[u].y * w;
+      acc0 += x0[u] * w;
+      acc1 += x1[u] * w;
+    }
+    M = m_new;
   }
+  // the split groups: lanes kCh apart hold the same row elements
+  float m_all = M;
+#pragma unroll
+  for (int off = kCh; off < 64; off <<= 1) m_all = fmaxf(m_all, __shfl_xor(m_all, off, 64));
+  const float f = M > -INFINITY ? exp2_fast(M - m_all) : 0.0f;
+  float v[9] = {Lsum * f,    acc0[0] * f, acc0[1] * f, acc0[2] * f, acc0[3] * f,
+                acc1[0] * f, acc1[1] * f, acc1[2] * f, acc1[3] * f};
+#pragma unroll
+  for (int off = kCh; off < 64; off <<= 1)
+#pragma unroll
+    for (int i = 0; i < 9; ++i) v[i] += __shfl_xor(v[i], off, 64);
+  if (sg != 0) return;
+  const float inv = v[0] > 0.0f ? 1.0f / v[0] : 0.0f;
+  const u32x4_t o = {pack_bf16x2(v[1] * inv, v[2] * inv), pack_bf16x2(v[3] * inv, v[4] * inv),
+                     pack_bf16x2(v[5] * inv, v[6] * inv), pack_bf16x2(v[7] * inv, v[8] * inv)};
+  const int hl = r / n, j = r - hl * n;
+  uint16_t* dst = a.out + static_cast<int64_t>(q0 + j) * a.o_ts +
+                  static_cast<int64_t>(hkv * a.G + hl) * a.o_hs + c * 8;
+  *reinterpret_cast<u32x4_t*>(dst) = o;
 }
 
 // Keys per split: a pure function of the launch shape, so the workspace can be sized without
 // reading seq_lens.  Aims at one block per CU (8-wave blocks) or two (4-wave blocks) for the
 // longest context, in whole rounds of 32-key tiles over the block's waves; a sequence longer
-// than one split is split, so shorter ones run whole.
+// than one split is split, so shorter ones run whole.  Contexts of up to kWholeRounds rounds
+// are not split however few the items are (1 sequence, 8 KV heads, bf16, 1 row, 400 keys: 9.0 us
+// whole, the merge launch alone costs 3); past that a split may be as short as one round (717
+// keys: 11.3 us whole, 11.9 in splits of two rounds, 9.7 of one; 4096 keys: 14.1 and 12.6).
+constexpr int kWholeRounds = 2;
 int target_blocks(int waves) { return waves == 8 ? 256 : 512; }
 
 int choose_split(int B, int Hkv, int max_seqlen_k, int waves) {
@@ -1105,7 +1116,7 @@ int choose_split(int B, int Hkv, int max_seqlen_k, int waves) {
   const int64_t gran = 32 * waves;
   int64_t per = (static_cast<int64_t>(max_seqlen_k) * items + target - 1) / target;
   per = ((per + gran - 1) / gran) * gran;
-  if (per < 2 * gran) per = 2 * gran;
+  if (max_seqlen_k <= kWholeRounds * gran && per < max_seqlen_k) per = kWholeRounds * gran;
   if (per > 65536) per = 65536;
   return static_cast<int>(per);
 }
@@ -1194,7 +1205,8 @@ int launch_rt(int RT, const AttnArgs& a, dim3 grid, hipStream_t s) {
   }
   int rc = coopt::check_launch("coopt_verify_attention");
   if (rc != COOPT_OK || a.max_splits <= 1) return rc;
-  hipLaunchKernelGGL((merge_kernel<D>), dim3(a.Hkv, a.B), dim3(kThreads), 0, s, a);
+  const int rows = a.Hkv * a.rmax, per = kThreads / 64;
+  hipLaunchKernelGGL((merge_kernel<D>), dim3((rows + per - 1) / per, a.B), dim3(kThreads), 0, s, a);
   return coopt::check_launch("coopt_verify_attention/merge");
 }
 

@@ -442,3 +442,28 @@ def test_windowed_call_needs_no_partials_workspace(dev):
     small = torch.empty(256, dtype=torch.uint8, device=dev)
     big = torch.empty(1 << 20, dtype=torch.uint8, device=dev)
     assert torch.equal(pool.run(workspace=small), pool.run(workspace=big))
+
+
+@pytest.mark.parametrize("kv", ["auto", "int8"])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("ctx,q_lens", [
+    ([0, 14, 15, 30, 31, 63, 254, 700], [1] * 8),     # last tiles of 1 to 32 keys, 1 to 3 splits
+    ([15, 250, 1999], [5, 1, 5]),                     # 8 splits
+    ([16001], [5]),                                   # 63 splits: eight merge rounds
+    ([3, 200], [33, 20]),                             # query windows
+])
+def test_rows_past_the_end_and_many_splits(dev, kv, D, ctx, q_lens):
+    """Cache rows past a sequence's end hold NaN (INT8: infinite scales) here; the tile loads
+    that cover them must not let them reach a result.  Tolerances as at the top."""
+    pool = Pool(ctx, q_lens, 32, 8, D, dev, kv=kv, seed=len(ctx) + D, slack=5)
+    written = torch.zeros(pool.kc.shape[:2], dtype=torch.bool, device=dev)
+    for b in range(len(ctx)):
+        pos = torch.arange(int(pool.seq_lens[b]), device=dev)
+        written[pool.table[b].long()[pos // pool.bs], pos % pool.bs] = True
+    for t in (pool.kc, pool.vc) if kv == "auto" else (pool.ks, pool.vs):
+        t[~written] = float("nan") if kv == "auto" else float("inf")
+    out = pool.run()
+    assert torch.isfinite(out.float()).all()
+    excess, mx, ulps = pool.max_err(out)
+    report(f"[stale rows {kv} D={D} ctx={ctx}] excess {excess:.4f} max-abs {mx:.4f} ulps {ulps:.2f}")
+    assert excess <= (TOL_BF16 if kv == "auto" else TOL_INT8)
