@@ -13,7 +13,8 @@ pass k_scale/v_scale; dequantisation is fused into the kernel.
 Supported: head_dim 64 or 128, any q_len.  Items of up to 64 rows per KV head, (Hq/Hkv) *
 max_seqlen_q <= 64 (speculative verify and decode), take the tuned path; longer ones (the
 prefill chunks engine/engine.py:414-420 mixes into the same batch) run in query windows of
-64/(Hq/Hkv) rows, one block per window and KV head -- correct at any length, not tuned.
+64/(Hq/Hkv) rows, one block per window and KV head -- or, for long chunks, of 128/(Hq/Hkv) rows in a
+kernel that stages K and V in LDS for the window's rows.
 """
 import math
 

@@ -16,9 +16,10 @@
 // cross-workgroup fence is needed.  A ragged batch with more (sequence, KV head) items than
 // one round of blocks holds runs on a 1-D grid whose blocks rank the sequences by length and
 // take the items longest first (plan_item), so its long sequences do not start last.
-// Items of more than 64 rows (prefill chunks of a mixed batch) are cut into query windows of
-// 64/G query rows -- each window is itself a sequence of those rows over the keys its last
-// row sees -- and run one unsplit block per (window, KV head): correct at any length.
+// Items of more than 64 rows (prefill chunks of a mixed batch) are cut into query windows -- each
+// window is itself a sequence of those rows over the keys its last row sees -- and run one
+// unsplit block per (window, KV head): windows of 64/G query tokens here, of 128/G in
+// prefill_attn_kernel, which takes the calls with long chunks.
 //
 // MFMA layout (v_mfma_f32_16x16x32_{bf16,f16}; lane l, g = l/16, m = l%16):
 //   scores  S^T[key][row] = sum_d K[key][d] Q[row][d]     A = K, B = Q^T
@@ -53,6 +54,8 @@
 // 8.3e6): it is set from the largest V scale seen so far and enters the softmax exponent, so
 // it cancels in o / l like the running max does.
 #include <math.h>
+
+#include <type_traits>
 
 #include "common.h"
 #include "kv_store.h"
@@ -99,8 +102,9 @@ struct AttnArgs {
   // Query windows (nwin > 0): a sequence's rows are taken qwin at a time, window w being rows
   // [w * qwin, (w + 1) * qwin) with the keys its last row sees -- on its own a sequence of
   // those rows, so the bottom-right causal mask stays exact.  1-D grid, block x = ((b * nwin)
-  // + w) * Hkv + hkv, one split per window.
+  // + w) * Hkv + hkv, one split per window (prefill_attn_kernel orders them itself).
   int qwin, nwin;
+  int prefill;  // host side: prefill_attn_kernel takes the windows
   // Fused qkv epilogue (coopt_verify_attention_qkv): qkv_mode 0 = q is given; 1 = bf16 qkv
   // projection rows; 2 = their fp32 split-K partials.  The block computes its own q rows
   // (RoPE'd, straight into LDS) and writes its KV head's new K/V to the cache first.
@@ -769,33 +773,32 @@ __global__ __launch_bounds__(64 * waves_for(RT), 1) void verify_attn_kernel(
   // one is computed) or, for large row counts, one at a time ----
   // Wave w takes tiles w, w + kWaves, w + 2 kWaves, ... (a fixed assignment keeps the result
   // bit-reproducible: each wave's sum covers the same keys on every call).  The split's partial
-  // last tile is one of them: loaded behind the full ones with a load of its own after the
-  // loop, it cost its wave a memory round trip (1 sequence, 717 keys, unsplit: 11.6 us, 11.3 in the loop).
+  // last tile is one of them: its loads are the last ones issued in the wave's loop, and it is
+  // computed behind the loop (loaded there as well, it cost its wave a memory round trip: 1
+  // sequence, 717 keys, unsplit: 11.6 us, 11.3 like this).
+  const int nfull = (k_end - k_begin) / kTileKeys;
+  const bool own_partial = nfull < ntiles && nfull % kWaves == wave;
+  const int tlast = own_partial ? nfull : nfull - 1;  // the last tile the wave may load
   auto pages = [&](int t, int64_t& p0, int64_t& p1) {
     const int kb = k_begin + t * kTileKeys;
     p0 = page_of(kb);
     p1 = page_of(kb + 16);
   };
-  // a loaded tile, before it is computed
-  auto prepare = [&](Raw& raw, int t) {
-    if (k_begin + (t + 1) * kTileKeys > k_end) clear_tail(raw, t);
-    vcheck(raw);
-  };
+  Raw bufA;
   if constexpr (DB) {
     // Loads inside the loop are unconditional (an index past the last tile repeats it,
     // already cached, and is never computed), so each compute waits only for its own
     // buffer's loads and the other buffer's stay in flight.
-    Raw bufA, bufB;
-    const int tlast = ntiles - 1;
+    Raw bufB;
     int tA = wave;
     int64_t nx0 = 0, nx1 = 0;  // pages of the wave's next tile to load
     // fused: a first tile holding keys this launch writes ([L - n, L)) loads after the barrier
     const bool defer = fused && k_begin + (tA + 1) * kTileKeys > L - n;
-    if (tA < ntiles && !defer) load_tile(bufA, tA, first_pg0, first_pg1);
+    if (tA <= tlast && !defer) load_tile(bufA, tA, first_pg0, first_pg1);
     stage_q();  // the Q loads complete while the first tile's are in flight
-    if (tA < ntiles && defer) load_tile(bufA, tA, first_pg0, first_pg1);
-    if (tA < ntiles) {
-      prepare(bufA, tA);
+    if (tA <= tlast && defer) load_tile(bufA, tA, first_pg0, first_pg1);
+    if (tA < nfull) {
+      vcheck(bufA);
       int tB = tA + kWaves;
       pages(min(tB, tlast), nx0, nx1);
       for (;;) {
@@ -803,28 +806,37 @@ __global__ __launch_bounds__(64 * waves_for(RT), 1) void verify_attn_kernel(
         const int tA2 = tB + kWaves;
         pages(min(tA2, tlast), nx0, nx1);
         compute_tile(bufA, tA);
-        if (tB >= ntiles) break;
-        prepare(bufB, tB);
+        if (tB >= nfull) {
+          bufA = bufB;
+          break;
+        }
+        vcheck(bufB);
         load_tile(bufA, min(tA2, tlast), nx0, nx1);
         const int tB2 = tA2 + kWaves;
         pages(min(tB2, tlast), nx0, nx1);
         compute_tile(bufB, tB);
-        if (tA2 >= ntiles) break;
-        prepare(bufA, tA2);
+        if (tA2 >= nfull) break;
+        vcheck(bufA);
         tA = tA2;
         tB = tB2;
       }
     }
   } else {
-    Raw buf;
     int64_t nx0 = first_pg0, nx1 = first_pg1;
     stage_q();
-    for (int t = wave; t < ntiles; t += kWaves) {
-      load_tile(buf, t, nx0, nx1);
-      if (t + kWaves < ntiles) pages(t + kWaves, nx0, nx1);
-      prepare(buf, t);
-      compute_tile(buf, t);
+    int t = wave;
+    for (; t < nfull; t += kWaves) {
+      load_tile(bufA, t, nx0, nx1);
+      if (t + kWaves <= tlast) pages(t + kWaves, nx0, nx1);
+      vcheck(bufA);
+      compute_tile(bufA, t);
     }
+    if (own_partial) load_tile(bufA, t, nx0, nx1);
+  }
+  if (own_partial) {
+    clear_tail(bufA, nfull);
+    vcheck(bufA);
+    compute_tile(bufA, nfull);
   }
   // ---- merge the waves ----
   // the wave's o and l are relative to 2^(m_run + e_v) (e_v = 0 for bf16 KV)
@@ -1100,6 +1112,473 @@ __global__ __launch_bounds__(kThreads) void merge_kernel(AttnArgs a) {
   *reinterpret_cast<u32x4_t*>(dst) = o;
 }
 
+// ---- items of many rows per KV head: prefill chunks, alone or in a mixed batch ----
+// A block of 4 waves takes one query window of one sequence and KV head: up to kPrefillRows rows
+// (kPrefillRows / G query tokens), 32 rows a wave.  The block walks the window's keys in stages of
+// 64, staged in LDS in MFMA operand order (a 16-byte chunk per lane and fragment: reads are
+// contiguous) and double-buffered: wave w stages sub-tile w's 16 keys, V transposed by byte
+// selects as build_va does, with two stages of global loads in flight.  Operands, softmax and
+// number formats are verify_attn_kernel's; Q lives in registers.  64 KB of LDS and 256 registers
+// let two blocks share a CU.
+// What bounds it: a wave's own instruction stream (about 165 VALU and 32 MFMA instructions a tile
+// and 32 rows) and, where windows are few, its chain per stage (1.3-2 us: staging 1.0 without the
+// tiles' work, the tiles 0.5-1.0).  Chunks of 1500 and 500 rows with 16 verify items of 5 rows
+// (bf16, 32/8 heads of 128, 30 GFLOP): 138 us on verify_attn_kernel's windows of 64 rows, whose
+// waves each read their own keys, 69 us here; INT8 190 and 82.
+// Tried: 64 keys per softmax (66-72 us, but 50 instead of 42 us for 2000 keys of a verify item alone,
+// which two waves share below), one stage of loads in flight with an L2 touch ahead (72).
+// Blocks take the windows with most keys first: window r from the end of every sequence before
+// window r + 1 of any (B <= kPlanSeqs; larger batches run in grid order).
+constexpr int kPrefillRows = 128;
+constexpr int kStageKeys = 64;
+
+template <int D, bool INT8>
+__global__ __launch_bounds__(256, 2) void prefill_attn_kernel(AttnArgs a) {
+  using Raw = RawTile<D, INT8>;
+  constexpr int kKs = D / 32, kDt = D / 16, kElt = Raw::kElt, kKVec = Raw::kKVec;
+  constexpr int kKFrag = kStageKeys / 16 * kKs, kVFrag = kStageKeys / 32 * kDt;
+  __shared__ u32x4_t lk[2][kKFrag * 64];
+  __shared__ u32x4_t lv[2][kVFrag * 64];
+  __shared__ uint16_t lsv[2][kStageKeys];
+  const int lane = threadIdx.x & 63, grp = lane >> 4, l16 = lane & 15;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  typedef const __attribute__((address_space(4))) int32_t* const_i32_ptr;
+
+  // ---- the block's window: sequence b, w-th window of its rows ----
+  const int x = static_cast<int>(blockIdx.x);
+  const int hkv = x % a.Hkv, k = x / a.Hkv;
+  int b, w;
+  if (a.B <= kPlanSeqs) {
+    int nw = 0;
+    if (lane < a.B) nw = min((max(a.cu[lane + 1] - a.cu[lane], 0) + a.qwin - 1) / a.qwin, a.nwin);
+    auto windows_to = [&](int r) {  // windows whose index from the end is below r
+      int v = min(nw, r);
+#pragma unroll
+      for (int off = 1; off < 64; off <<= 1) v += __shfl_xor(v, off, 64);
+      return __builtin_amdgcn_readfirstlane(v);
+    };
+    int lo = 0, hi = a.nwin;  // the largest r with windows_to(r) <= k
+    if (k >= windows_to(hi)) return;
+    while (hi - lo > 1) {
+      const int mid = (lo + hi) >> 1;
+      if (windows_to(mid) <= k) lo = mid;
+      else hi = mid;
+    }
+    const int at = k - windows_to(lo);  // the at-th sequence with more than lo windows
+    const uint64_t has = __builtin_amdgcn_ballot_w64(nw > lo);
+    const uint64_t mine = __builtin_amdgcn_ballot_w64(
+        nw > lo && static_cast<int>(__popcll(has & ((uint64_t{1} << lane) - 1))) == at);
+    b = __builtin_amdgcn_readfirstlane(__ffsll(static_cast<unsigned long long>(mine)) - 1);
+    w = __builtin_amdgcn_readlane(nw, b) - 1 - lo;
+  } else {
+    b = k / a.nwin;
+    w = a.nwin - 1 - (k - b * a.nwin);
+  }
+  const const_i32_ptr cuc = (const_i32_ptr)a.cu;
+  const const_i32_ptr slc = (const_i32_ptr)a.seq_lens;
+  const int c0 = cuc[b], nall = cuc[b + 1] - c0, j0 = w * a.qwin;
+  const int n = min(max(nall - j0, 0), a.qwin);
+  if (n <= 0) return;
+  const int q0 = c0 + j0;
+  const int L = min(static_cast<int>(slc[b]), a.max_seqlen_k) - (nall - j0 - n);
+  const int R = a.G * n;
+  const const_i32_ptr table = (const_i32_ptr)(a.bt + static_cast<int64_t>(b) * a.bt_stride);
+  const int bs_mask = (1 << a.bs_shift) - 1;
+  // Windows of at most 64 rows (verify items, the end of a chunk): two waves a row group, each
+  // with one of a stage's two tiles, merged at the end.
+  const bool pair = R <= 64;
+  const int row0 = (pair ? wave & 1 : wave) * 32;  // row r of the window: query token r / G, head r % G
+  const bool idle = row0 >= R;
+
+  // ---- Q operands and causal limits ----
+  u32x4_t qop[2][kKs];
+  int lim[2];
+#pragma unroll
+  for (int rt = 0; rt < 2; ++rt) {
+    const int r = row0 + rt * 16 + l16;
+    const int j = r / a.G, hl = r - j * a.G;
+    lim[rt] = r < R ? L - n + j : -1;
+    const int64_t qoff = static_cast<int64_t>(q0 + j) * a.q_ts + static_cast<int64_t>(hkv * a.G + hl) * a.q_hs;
+#pragma unroll
+    for (int ks = 0; ks < kKs; ++ks) {
+      const int d = INT8 ? 64 * (ks >> 1) + 16 * grp + 8 * (ks & 1) : 32 * ks + 8 * grp;
+      qop[rt][ks] = r < R ? *reinterpret_cast<const u32x4_t*>(a.q + qoff + d) : u32x4_t{0, 0, 0, 0};
+    }
+  }
+  const int first_lim = L - n + row0 / a.G;                        // of the wave's first row
+  const int last_lim = L - n + (min(row0 + 32, R) - 1) / a.G;      // and of its last
+
+  f32x4_t o[2][kDt];
+  float m_run[2], l_run[2];
+#pragma unroll
+  for (int rt = 0; rt < 2; ++rt) {
+    m_run[rt] = -INFINITY;
+    l_run[rt] = 0.0f;
+#pragma unroll
+    for (int dt = 0; dt < kDt; ++dt) o[rt][dt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  }
+  int e_v = 0;  // INT8: the V-scale reference exponent, as in verify_attn_kernel
+  bool ev_set = false;
+
+  // ---- staging: wave w takes the K and V of sub-tile w, 16 of a stage's 64 keys ----
+  const int stages = L > 0 ? (L + kStageKeys - 1) / kStageKeys : 0;
+  const int tile = wave >> 1, half = wave & 1;  // its 32-key tile, and which half of it
+  const unsigned char* const kbase = static_cast<const unsigned char*>(a.kc);
+  const unsigned char* const vbase = static_cast<const unsigned char*>(a.vc);
+  const int64_t head_off = static_cast<int64_t>(hkv) * a.c_hs;
+  const int64_t shead_off = static_cast<int64_t>(hkv) * a.s_hs;
+  const int c_ts = static_cast<int>(a.c_ts), s_ts = static_cast<int>(a.s_ts);
+  const uint32_t k_lane = kElt * l16 * c_ts + 16 * grp;
+  const uint32_t v_lane = kElt * (grp * 4 * c_ts + l16 * kDt);
+  auto page_of = [&](int s) {
+    return clamp_page(table[min(s * kStageKeys + wave * 16, L - 1) >> a.bs_shift], a.num_blocks);
+  };
+  struct Staged {
+    u32x4_t k[kKVec];             // 64 bytes apart of key l16
+    uint32_t v[4][Raw::kVWords];  // kDt elements of keys 4 grp .. 4 grp + 3
+    uint32_t ks;                  // INT8: the scales of those keys
+    u32x2_t vs;
+  };
+  auto load_stage = [&](Staged& st, int s, int64_t pg) {
+    const int tok0 = (s * kStageKeys + wave * 16) & bs_mask;
+    const int64_t r = pg * a.c_bs + head_off + static_cast<int64_t>(tok0) * c_ts;
+    if constexpr (INT8) {
+      const int64_t rs = pg * a.s_bs + shead_off;
+      st.ks = a.ks[rs + (tok0 + l16) * s_ts];
+      uint32_t h[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) h[i] = a.vs[rs + (tok0 + grp * 4 + i) * s_ts];
+      st.vs = u32x2_t{h[0] | (h[1] << 16), h[2] | (h[3] << 16)};
+    }
+#pragma unroll
+    for (int c = 0; c < kKVec; ++c)
+      st.k[c] = *reinterpret_cast<const u32x4_t*>(kbase + kElt * r + 64 * c + k_lane);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const unsigned char* src = vbase + kElt * (r + i * c_ts) + v_lane;
+      if constexpr (Raw::kVWords == 4) {
+        const u32x4_t v = *reinterpret_cast<const u32x4_t*>(src);
+        st.v[i][0] = v[0]; st.v[i][1] = v[1]; st.v[i][2] = v[2]; st.v[i][3] = v[3];
+      } else if constexpr (Raw::kVWords == 2) {
+        const u32x2_t v = *reinterpret_cast<const u32x2_t*>(src);
+        st.v[i][0] = v[0]; st.v[i][1] = v[1];
+      } else {
+        st.v[i][0] = *reinterpret_cast<const uint32_t*>(src);
+      }
+    }
+  };
+  constexpr uint32_t k64 = 0x64646464u;  // fp16 exponent bytes of 1024
+  auto store_stage = [&](const Staged& st, int s) {
+    const int buf = s & 1;
+    u32x4_t* const kd = &lk[buf][wave * kKs * 64 + lane];
+    if constexpr (INT8) {
+      const float sk = f16_to_f32(static_cast<uint16_t>(st.ks));
+      const float skb = -1152.0f * sk;
+#pragma unroll
+      for (int ks = 0; ks < kKs; ++ks) {
+        u32x4_t kop;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const uint32_t ux = st.k[ks >> 1][(ks & 1) * 2 + h] ^ 0x80808080u;
+          kop[2 * h] = dequant_pair(__builtin_amdgcn_perm(k64, ux, 0x04010400u), sk, skb);
+          kop[2 * h + 1] = dequant_pair(__builtin_amdgcn_perm(k64, ux, 0x04030402u), sk, skb);
+        }
+        kd[ks * 64] = kop;
+      }
+    } else {
+#pragma unroll
+      for (int c = 0; c < kKVec; ++c) kd[c * 64] = st.k[c];
+    }
+    // keys past the window's last: zero values and scales (the rows may never have been written)
+    const int left = L - (s * kStageKeys + wave * 16) - grp * 4;
+    uint32_t vx[4][Raw::kVWords];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int e = 0; e < Raw::kVWords; ++e) vx[j][e] = st.v[j][e] ^ (INT8 ? 0x80808080u : 0u);
+    if (L - (s * kStageKeys + wave * 16) < 16) {  // uniform
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int e = 0; e < Raw::kVWords; ++e)
+          if (j >= left) vx[j][e] = INT8 ? 0x80808080u : 0u;
+    }
+    if constexpr (INT8) {
+      u32x2_t vs = st.vs;
+      vs[0] &= (left > 0 ? 0xffffu : 0u) | (left > 1 ? 0xffff0000u : 0u);
+      vs[1] &= (left > 2 ? 0xffffu : 0u) | (left > 3 ? 0xffff0000u : 0u);
+      if (l16 == 0) *reinterpret_cast<u32x2_t*>(&lsv[buf][wave * 16 + grp * 4]) = vs;
+    }
+    // fragment dt of the tile: 8 keys of d-tile dt per lane, this wave's 4 in its half's 8 bytes
+    u32x2_t* const vd = reinterpret_cast<u32x2_t*>(&lv[buf][tile * kDt * 64 + lane]) + half;
+    if constexpr (INT8) {
+#pragma unroll
+      for (int e = 0; e < Raw::kVWords; ++e) {
+        u32x2_t va[4];
+#pragma unroll
+        for (int e2 = 0; e2 < 2; ++e2) {
+          const uint32_t lo = __builtin_amdgcn_perm(vx[2 * e2 + 1][e], vx[2 * e2][e], 0x05010400u);
+          const uint32_t hi = __builtin_amdgcn_perm(vx[2 * e2 + 1][e], vx[2 * e2][e], 0x07030602u);
+          va[0][e2] = codes_f16x2(__builtin_amdgcn_perm(k64, lo, 0x04010400u));
+          va[1][e2] = codes_f16x2(__builtin_amdgcn_perm(k64, lo, 0x04030402u));
+          va[2][e2] = codes_f16x2(__builtin_amdgcn_perm(k64, hi, 0x04010400u));
+          va[3][e2] = codes_f16x2(__builtin_amdgcn_perm(k64, hi, 0x04030402u));
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) vd[(4 * e + q) * 128] = va[q];
+      }
+    } else {
+#pragma unroll
+      for (int dt = 0; dt < kDt; ++dt) {
+        u32x2_t va;
+#pragma unroll
+        for (int e2 = 0; e2 < 2; ++e2)
+          va[e2] = __builtin_amdgcn_perm(vx[2 * e2 + 1][dt >> 1], vx[2 * e2][dt >> 1],
+                                         (dt & 1) ? 0x07060302u : 0x05040100u);
+        vd[dt * 128] = va;
+      }
+    }
+  };
+
+  // ---- one 32-key tile of a stage for the wave's 32 rows ----
+  constexpr int kSub = 2;  // 16-key sub-tiles
+  auto compute_tile = [&](int s, int t0) {
+    const int kb = s * kStageKeys + 32 * t0, buf = s & 1;
+    const u32x4_t* const fk = &lk[buf][t0 * 2 * kKs * 64 + lane];
+    const u32x4_t* const fv = &lv[buf][t0 * kDt * 64 + lane];
+    f32x4_t acc[2][kSub];
+#pragma unroll
+    for (int rt = 0; rt < 2; ++rt)
+#pragma unroll
+      for (int kt = 0; kt < kSub; ++kt) acc[rt][kt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int ks = 0; ks < kKs; ++ks)
+#pragma unroll
+      for (int kt = 0; kt < kSub; ++kt) {
+        const u32x4_t kop = fk[(kt * kKs + ks) * 64];
+#pragma unroll
+        for (int rt = 0; rt < 2; ++rt) acc[rt][kt] = mfma_bf16(kop, qop[rt][ks], acc[rt][kt]);
+      }
+    // two k-steps' fragments ahead of the MFMAs that take them (0x100: LDS reads, 8: MFMAs)
+    __builtin_amdgcn_sched_group_barrier(0x100, 2 * kSub, 0);
+#pragma unroll
+    for (int ks = 0; ks < kKs; ++ks) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 2 * kSub, 0);
+      if (ks + 2 < kKs) __builtin_amdgcn_sched_group_barrier(0x100, kSub, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    // V's fragments, read under the softmax
+    u32x4_t va[kDt];
+#pragma unroll
+    for (int dt = 0; dt < kDt; ++dt) va[dt] = fv[dt * 64];
+    u32x2_t vs[kSub];
+    if constexpr (INT8) {
+#pragma unroll
+      for (int kt = 0; kt < kSub; ++kt)
+        vs[kt] = *reinterpret_cast<const u32x2_t*>(&lsv[buf][t0 * 32 + kt * 16 + grp * 4]);
+      uint32_t wv = 0;
+#pragma unroll
+      for (int kt = 0; kt < kSub; ++kt) wv = max_u16x2(wv, max_u16x2(vs[kt][0], vs[kt][1]));
+      const uint32_t smax = min(max(wv & 0xffffu, wv >> 16), 0x7bffu);
+      const uint32_t thr = !ev_set ? 0u
+                           : (e_v + 7 >= 16 ? 0x7c00u : static_cast<uint32_t>(e_v + 7 + 15) << 10);
+      if (__builtin_amdgcn_ballot_w64(smax > thr)) {
+        uint32_t wm = smax;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1)
+          wm = max(wm, static_cast<uint32_t>(__shfl_xor(static_cast<int>(wm), off, 64)));
+        const int e_new = __builtin_amdgcn_readfirstlane(static_cast<int>(wm >> 10) - 21);
+        const float f = exp2_fast(static_cast<float>(e_v - e_new));
+#pragma unroll
+        for (int rt = 0; rt < 2; ++rt) {
+          l_run[rt] *= f;
+#pragma unroll
+          for (int dt = 0; dt < kDt; ++dt) o[rt][dt] *= f;
+        }
+        e_v = e_new;
+        ev_set = true;
+      }
+    }
+    // bf16 probabilities: the reference is the running maximum itself (no slack), so the largest
+    // one is exactly 1; with the slack and unrounded sums one reference for all keys was 2 %
+    // further from 64 bits than verify_attn_kernel's one per wave (2.10e-3 against 2.05e-3 relative
+    // in the batch above; like this 2.01e-3)
+    constexpr float kSlack = INT8 ? 8.0f : 0.0f;
+    if (kb + 31 > first_lim) {  // some row does not see every key (those past L are past it)
+#pragma unroll
+      for (int rt = 0; rt < 2; ++rt)
+#pragma unroll
+        for (int kt = 0; kt < kSub; ++kt)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (kb + kt * 16 + grp * 4 + i > lim[rt]) acc[rt][kt][i] = -INFINITY;
+    }
+    float m_tile[2];
+    bool raise_any = false;
+#pragma unroll
+    for (int rt = 0; rt < 2; ++rt) {
+      float tmax = -INFINITY;
+#pragma unroll
+      for (int kt = 0; kt < kSub; ++kt)
+        tmax = fmaxf(tmax, fmaxf(fmaxf(acc[rt][kt][0], acc[rt][kt][1]), fmaxf(acc[rt][kt][2], acc[rt][kt][3])));
+      tmax = max_xor32(max_xor16(tmax));
+      m_tile[rt] = tmax * a.scale_log2;
+      raise_any |= m_tile[rt] > m_run[rt] + kSlack;
+    }
+    if (__builtin_amdgcn_ballot_w64(raise_any)) {
+#pragma unroll
+      for (int rt = 0; rt < 2; ++rt) {
+        const bool raise = m_tile[rt] > m_run[rt] + kSlack;
+        const float m_new = raise ? m_tile[rt] : m_run[rt];
+        const float alpha = raise ? exp2_fast(m_run[rt] - m_new) : 1.0f;
+        l_run[rt] *= alpha;
+#pragma unroll
+        for (int dt = 0; dt < kDt; ++dt) o[rt][dt] *= alpha;
+        m_run[rt] = m_new;
+      }
+    }
+    u32x4_t pb[2][kSub / 2];
+#pragma unroll
+    for (int rt = 0; rt < 2; ++rt) {
+      const float m_use = (m_run[rt] == -INFINITY ? 0.0f : m_run[rt]) + (INT8 ? static_cast<float>(e_v) : 0.0f);
+#pragma unroll
+      for (int kt = 0; kt < kSub; ++kt) {
+        float pr[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) pr[i] = exp2_fast(fmaf(acc[rt][kt][i], a.scale_log2, -m_use));
+        if constexpr (INT8) {
+          l_run[rt] += (pr[0] + pr[1]) + (pr[2] + pr[3]);
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            pr[i] *= f16_to_f32(static_cast<uint16_t>(vs[kt][i >> 1] >> (16 * (i & 1))));
+          pb[rt][kt >> 1][2 * (kt & 1)] = pack_f16x2(pr[0], pr[1]);
+          pb[rt][kt >> 1][2 * (kt & 1) + 1] = pack_f16x2(pr[2], pr[3]);
+        } else {
+          const uint32_t p0 = pack_bf16x2(pr[0], pr[1]), p1 = pack_bf16x2(pr[2], pr[3]);
+          pb[rt][kt >> 1][2 * (kt & 1)] = p0;
+          pb[rt][kt >> 1][2 * (kt & 1) + 1] = p1;
+        }
+      }
+    }
+    if constexpr (!INT8) {
+      // l: the sum of the rounded probabilities (their common rounding cancels in o / l), as a
+      // product with ones
+      constexpr uint32_t kOnes = 0x3f803f80u;
+      const u32x4_t ones = {kOnes, kOnes, kOnes, kOnes};
+#pragma unroll
+      for (int rt = 0; rt < 2; ++rt) {
+        f32x4_t sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int t = 0; t < kSub / 2; ++t) sum = mfma_bf16(ones, pb[rt][t], sum);
+        l_run[rt] += sum[0];
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int dt = 0; dt < kDt; ++dt) {
+#pragma unroll
+      for (int rt = 0; rt < 2; ++rt)
+        o[rt][dt] = INT8 ? mfma_f16(va[dt], pb[rt][0], o[rt][dt]) : mfma_bf16(va[dt], pb[rt][0], o[rt][dt]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+
+  // Two register sets: stage s + 2 loads while stage s is computed and stage s + 1 waits in the
+  // other set.  Loads past the last stage repeat it (cached), so no load sits under a branch.
+  if (stages > 0) {
+    Staged sa, sb;
+    const int last = stages - 1;
+    int64_t pg = page_of(0);
+    auto load = [&](Staged& st, int s) {
+      const int64_t now = pg;
+      pg = page_of(min(s + 1, last));  // looked up a stage ahead
+      load_stage(st, min(s, last), now);
+    };
+    auto compute = [&](int s) {
+      if (idle) return;
+#pragma unroll 1
+      for (int t = pair ? tile : 0; t <= (pair ? tile : 1); ++t)
+        if (s * kStageKeys + 32 * t <= last_lim) compute_tile(s, t);
+    };
+    load(sa, 0);
+    load(sb, 1);
+    store_stage(sa, 0);
+    __syncthreads();
+    int s = 0;
+    for (; s + 2 <= last; s += 2) {
+      load(sa, s + 2);
+      compute(s);
+      store_stage(sb, s + 1);
+      __syncthreads();
+      load(sb, s + 3);
+      compute(s + 1);
+      store_stage(sa, s + 2);
+      __syncthreads();
+    }
+    compute(s);
+    if (s < last) {
+      store_stage(sb, s + 1);
+      __syncthreads();
+      compute(s + 1);
+    }
+  }
+  // bf16: every lane of a row's column holds its whole sum already
+  if constexpr (INT8) {
+#pragma unroll
+    for (int rt = 0; rt < 2; ++rt) {
+      l_run[rt] = add_xor32(add_xor16(l_run[rt]));
+      m_run[rt] += static_cast<float>(e_v);  // o and l are relative to 2^(m_run + e_v)
+    }
+  }
+  if (pair) {  // waves 2 and 3 hand their sums to waves 0 and 1
+    constexpr int kWords = 2 * kDt + 1;
+    static_assert(kWords <= 2 * kKFrag && kWords <= 2 * kVFrag, "a wave's sums fit one staging array");
+    u32x4_t* const xch = (wave & 1 ? &lv[0][0] : &lk[0][0]) + lane;
+    __syncthreads();
+    if (tile == 1 && !idle) {
+#pragma unroll
+      for (int rt = 0; rt < 2; ++rt)
+#pragma unroll
+        for (int dt = 0; dt < kDt; ++dt) xch[(rt * kDt + dt) * 64] = __builtin_bit_cast(u32x4_t, o[rt][dt]);
+      xch[2 * kDt * 64] = u32x4_t{__float_as_uint(m_run[0]), __float_as_uint(l_run[0]),
+                                  __float_as_uint(m_run[1]), __float_as_uint(l_run[1])};
+    }
+    __syncthreads();
+    if (tile == 1 || idle) return;
+    const u32x4_t ml = xch[2 * kDt * 64];
+#pragma unroll
+    for (int rt = 0; rt < 2; ++rt) {
+      const float m2 = __uint_as_float(ml[2 * rt]), l2 = __uint_as_float(ml[2 * rt + 1]);
+      const float M = fmaxf(m_run[rt], m2);
+      const float f1 = m_run[rt] > -INFINITY ? exp2_fast(m_run[rt] - M) : 0.0f;
+      const float f2 = m2 > -INFINITY ? exp2_fast(m2 - M) : 0.0f;
+      l_run[rt] = l_run[rt] * f1 + l2 * f2;
+#pragma unroll
+      for (int dt = 0; dt < kDt; ++dt)
+        o[rt][dt] = o[rt][dt] * f1 + __builtin_bit_cast(f32x4_t, xch[(rt * kDt + dt) * 64]) * f2;
+    }
+  }
+  // ---- normalise and write: lane's row l16 of each row tile, d = (4 grp + i) * kDt + dt ----
+#pragma unroll
+  for (int rt = 0; rt < 2; ++rt) {
+    const float inv = l_run[rt] > 0.0f ? 1.0f / l_run[rt] : 0.0f;
+    const int r = row0 + rt * 16 + l16;
+    if (r >= R) continue;
+    const int j = r / a.G, hl = r - j * a.G;
+    uint16_t* const row = a.out + static_cast<int64_t>(q0 + j) * a.o_ts + static_cast<int64_t>(hkv * a.G + hl) * a.o_hs;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      uint16_t* dst = row + (grp * 4 + i) * kDt;
+      uint32_t v[kDt / 2];
+#pragma unroll
+      for (int e = 0; e < kDt / 2; ++e) v[e] = pack_bf16x2(o[rt][2 * e][i] * inv, o[rt][2 * e + 1][i] * inv);
+      if constexpr (kDt == 8) *reinterpret_cast<u32x4_t*>(dst) = u32x4_t{v[0], v[1], v[2], v[3]};
+      else *reinterpret_cast<u32x2_t*>(dst) = u32x2_t{v[0], v[1]};
+    }
+  }
+}
+
 // Keys per split: a pure function of the launch shape, so the workspace can be sized without
 // reading seq_lens.  Aims at one block per CU (8-wave blocks) or two (4-wave blocks) for the
 // longest context, in whole rounds of 32-key tiles over the block's waves; a sequence longer
@@ -1131,22 +1610,31 @@ struct AttnShape {
   int split, max_splits;
   int rmax;        // rows per (item, KV head): G * max_seqlen_q, or G * qwin when windowed
   int qwin, nwin;  // windowed: rows per window and windows per sequence (else 0, 0)
+  bool prefill;    // windowed, by prefill_attn_kernel
 };
 
 constexpr int kMaxRows = 64;
+// Which of the two takes a windowed call.  prefill_attn_kernel has the higher rate,
+// verify_attn_kernel the shorter chain per window (its four waves share a window's keys), so the
+// first takes calls that may hold many windows: chunks of 2048 rows (512 tokens at G = 4) or
+// more, or 32 sequences with items of 256 rows.  bf16, 32/8 heads of 128, old / new us: chunks of
+// 1500 + 500 rows and 16 verify items 138 / 69, 512 + 17 and 20 66 / 27, 2048 + 1000 and 32 388 / 182,
+// 600 + 100 and 2 65 / 68, 64 + 17 and 32 109 / 60; below the line 300 + 100 and 8 70 / 80, 260 + 17 and
+// 2 52 / 66, 17 + 17 and 4 35 / 64.
+constexpr int kPrefillFrom = 2048, kPrefillFromMany = 256, kManySeqs = 32;
 
 AttnShape attn_shape(int B, int G, int Hkv, int max_seqlen_q, int max_seqlen_k) {
   AttnShape s{};
   if (G * static_cast<int64_t>(max_seqlen_q) > kMaxRows) {
-    // prefill-sized rows (a chunk of a mixed batch, a long catch-up): windows of kMaxRows / G
-    // rows, each one unsplit block -- correct at any length, not tuned for throughput
-    s.qwin = kMaxRows / G;
+    // longer items run in query windows of kMaxRows (verify_attn_kernel: a wave's tiles are its
+    // own, which suits few windows) or kPrefillRows rows (prefill_attn_kernel)
+    s.prefill = G * static_cast<int64_t>(max_seqlen_q) >= (B >= kManySeqs ? kPrefillFromMany : kPrefillFrom);
+    s.qwin = (s.prefill ? kPrefillRows : kMaxRows) / G;
     s.nwin = (max_seqlen_q + s.qwin - 1) / s.qwin;
     s.rmax = G * s.qwin;
     const int gran = 32 * waves_for((s.rmax + 15) / 16);
     s.split = static_cast<int>((static_cast<int64_t>(max_seqlen_k) + gran - 1) / gran * gran);
     s.max_splits = 1;
-    s.plan = false;
     return s;
   }
   s.rmax = G * max_seqlen_q;
@@ -1212,6 +1700,11 @@ int launch_rt(int RT, const AttnArgs& a, dim3 grid, hipStream_t s) {
 
 template <int D>
 int launch_d(bool int8, bool sc, int RT, const AttnArgs& a, dim3 grid, hipStream_t s) {
+  if (a.prefill) {
+    if (int8) hipLaunchKernelGGL((prefill_attn_kernel<D, true>), grid, dim3(256), 0, s, a);
+    else hipLaunchKernelGGL((prefill_attn_kernel<D, false>), grid, dim3(256), 0, s, a);
+    return coopt::check_launch("coopt_verify_attention/prefill");
+  }
   if (!int8) return launch_rt<D, false, false>(RT, a, grid, s);
   return sc ? launch_rt<D, true, true>(RT, a, grid, s) : launch_rt<D, true, false>(RT, a, grid, s);
 }
@@ -1340,6 +1833,7 @@ int verify_attention_impl(const char* who, const FusedQkv* fz, int kv_dtype, con
   a.rmax = shape.rmax;
   a.qwin = shape.qwin;
   a.nwin = shape.nwin;
+  a.prefill = shape.prefill;
   a.split = shape.split;
   a.max_splits = shape.max_splits;
   a.B = B;

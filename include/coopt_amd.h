@@ -242,9 +242,11 @@ int coopt_kv_copy_blocks(const int64_t* regions, int num_regions, const int64_t*
  *   Query rows: up to 64 rows per (sequence, KV head), i.e. (Hq/Hkv) * max_seqlen_q <= 64
  *   (speculative verify and decode), run on the tuned path (contexts split over blocks).
  *   Longer items -- the prefill chunks the engine mixes into one batch with its verify items
- *   (engine/engine.py:414-420), or a long draft catch-up -- run in query windows of
- *   64/(Hq/Hkv) rows, each window one block over the keys its last row sees: correct at any
- *   length, not tuned for throughput (B * windows * Hkv < 2^24 blocks).  Callers must keep seq_lens <= max_seqlen_k, q rows per sequence
+ *   (engine/engine.py:414-420), or a long draft catch-up -- run in query windows, each one
+ *   block over the keys its last row sees: of 64/(Hq/Hkv) rows, or, with chunks of 2048 rows
+ *   per KV head (or 256 in batches of 32 sequences) and more, of 128/(Hq/Hkv) rows in a kernel
+ *   that stages K and V in LDS (B * windows * Hkv < 2^24 blocks).
+ *   Callers must keep seq_lens <= max_seqlen_k, q rows per sequence
  *   <= max_seqlen_q and block ids in [0, num_blocks); the kernel clamps all three so a
  *   malformed call yields wrong rows but never an access outside its buffers.
  *   workspace: coopt_verify_attention_workspace() bytes (see above).

@@ -467,3 +467,29 @@ def test_rows_past_the_end_and_many_splits(dev, kv, D, ctx, q_lens):
     excess, mx, ulps = pool.max_err(out)
     report(f"[stale rows {kv} D={D} ctx={ctx}] excess {excess:.4f} max-abs {mx:.4f} ulps {ulps:.2f}")
     assert excess <= (TOL_BF16 if kv == "auto" else TOL_INT8)
+
+
+@pytest.mark.parametrize("kv,D,G,ctx,q_lens,bs", [
+    ("auto", 128, 4, [0, 37, 900, 5], [513, 1, 5, 64], 16),       # 17 windows, the last of 1 row
+    ("int8", 128, 4, [0, 37, 900, 5], [513, 1, 5, 65], 16),
+    ("auto", 64, 1, [130, 0], [2049, 128], 32),                   # windows of 128 query tokens
+    ("int8", 64, 8, [63, 64, 1], [257, 16, 17], 64),              # of 16
+    ("int8", 128, 4, [10] * 3 + [300] * 67, [64, 1, 33] + [2] * 67, 16),  # 70 sequences: grid order
+    ("auto", 64, 4, list(range(0, 320, 10)), [64] * 32, 16),      # 32 sequences of 256 rows
+])
+def test_long_chunks_match_the_oracle(dev, kv, D, G, ctx, q_lens, bs):
+    """The prefill kernel (2048 rows per KV head, or 256 with 32 sequences): window and stage
+    remainders, mixed batches, stale rows past the end.  Tolerances as at the top."""
+    pool = Pool(ctx, q_lens, 4 * G, 4, D, dev, kv=kv, bs=bs, seed=D + G, slack=2)
+    for t in (pool.kc, pool.vc) if kv == "auto" else (pool.ks, pool.vs):
+        b = len(ctx) - 1                                          # rows past one sequence's end
+        L = int(pool.seq_lens[b])
+        if L % bs:
+            t[pool.table[b].long()[L // bs], L % bs:] = float("nan")
+    out = pool.run()
+    assert torch.isfinite(out.float()).all()
+    assert torch.equal(out, pool.run())
+    seqs = list(range(min(4, len(ctx)))) + [len(ctx) - 1]
+    excess, mx, ulps = pool.max_err(out, sorted(set(seqs)))
+    report(f"[long chunks {kv} D={D} G={G}] excess {excess:.4f} max-abs {mx:.4f} ulps {ulps:.2f}")
+    assert excess <= (TOL_BF16 if kv == "auto" else TOL_INT8)
