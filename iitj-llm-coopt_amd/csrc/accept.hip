@@ -135,6 +135,7 @@ struct Args {
   const float* u_res;
   int32_t* acc_len;
   int32_t* out_tok;
+  int64_t* out_tok64;  // coopt_sample64: the tokens go here instead
   float* margin;
   float inv_t;
   int draft_probs;
@@ -1396,7 +1397,8 @@ __global__ __launch_bounds__(kThreads) void sample_select_kernel(Args a, float* 
       pick = sh_last >= 0 ? sh_last : lo;
       pm = 0.0f;
     }
-    a.out_tok[static_cast<int64_t>(b) * (a.gmax + 1)] = pick;
+    if (a.out_tok64) a.out_tok64[b] = pick;
+    else a.out_tok[static_cast<int64_t>(b) * (a.gmax + 1)] = pick;
     if (a.acc_len) a.acc_len[b] = 0;  // null for coopt_sample (tokens only)
     if (a.margin) a.margin[b] = pm;
   }
@@ -1606,9 +1608,11 @@ extern "C" int coopt_softmax(int logits_dtype, const void* logits, int64_t in_st
   return coopt::check_launch("coopt_softmax");
 }
 
-extern "C" int coopt_sample(int logits_dtype, const void* logits, int64_t row_stride, int N, int V,
-                            float temperature, const float* uniforms, int32_t* tokens,
-                            float* margin, float* probs, int64_t probs_stride, void* workspace,
+namespace {
+
+int sample_impl(int logits_dtype, const void* logits, int64_t row_stride, int N, int V,
+                float temperature, const float* uniforms, int32_t* tokens, int64_t* tokens64,
+                float* margin, float* probs, int64_t probs_stride, void* workspace,
                             size_t workspace_bytes, coopt_stream_t stream) {
   COOPT_REQUIRE(logits_dtype == COOPT_DT_F32 || logits_dtype == COOPT_DT_BF16,
                 "logits_dtype must be F32 or BF16");
@@ -1616,7 +1620,7 @@ extern "C" int coopt_sample(int logits_dtype, const void* logits, int64_t row_st
   COOPT_REQUIRE(temperature > 0.0f, "temperature must be > 0 (greedy rows: coopt_accept_sample)");
   COOPT_REQUIRE(!probs || probs_stride >= V, "probs_stride < V");
   if (N == 0) return COOPT_OK;
-  COOPT_REQUIRE(logits && uniforms && tokens && workspace, "null pointer");
+  COOPT_REQUIRE(logits && uniforms && (tokens || tokens64) && workspace, "null pointer");
   const size_t need = coopt_accept_sample_workspace(N, 0, V);
   if (workspace_bytes < need) {
     coopt::set_error("coopt_sample: workspace too small");
@@ -1629,6 +1633,7 @@ extern "C" int coopt_sample(int logits_dtype, const void* logits, int64_t row_st
   a.tgt_stride = row_stride;
   a.u_res = uniforms;
   a.out_tok = tokens;
+  a.out_tok64 = tokens64;
   a.margin = margin;
   a.inv_t = 1.0f / temperature;
   a.vec_t = coopt::aligned16(logits) && row_stride % (bf16 ? 8 : 4) == 0;
@@ -1641,6 +1646,24 @@ extern "C" int coopt_sample(int logits_dtype, const void* logits, int64_t row_st
   auto s = static_cast<hipStream_t>(stream);
   return bf16 ? launch_all<true>(a, false, s, probs, probs_stride, vec_out)
               : launch_all<false>(a, false, s, probs, probs_stride, vec_out);
+}
+
+}  // namespace
+
+extern "C" int coopt_sample(int logits_dtype, const void* logits, int64_t row_stride, int N, int V,
+                            float temperature, const float* uniforms, int32_t* tokens,
+                            float* margin, float* probs, int64_t probs_stride, void* workspace,
+                            size_t workspace_bytes, coopt_stream_t stream) {
+  return sample_impl(logits_dtype, logits, row_stride, N, V, temperature, uniforms, tokens, nullptr, margin,
+                     probs, probs_stride, workspace, workspace_bytes, stream);
+}
+
+extern "C" int coopt_sample64(int logits_dtype, const void* logits, int64_t row_stride, int N, int V,
+                            float temperature, const float* uniforms, int64_t* tokens,
+                            float* margin, float* probs, int64_t probs_stride, void* workspace,
+                            size_t workspace_bytes, coopt_stream_t stream) {
+  return sample_impl(logits_dtype, logits, row_stride, N, V, temperature, uniforms, nullptr, tokens, margin,
+                     probs, probs_stride, workspace, workspace_bytes, stream);
 }
 
 extern "C" int coopt_sample_probs(int logits_dtype, const void* logits, int64_t in_stride, int B,

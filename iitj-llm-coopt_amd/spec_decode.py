@@ -180,7 +180,7 @@ def sample(logits: torch.Tensor, temperature: float, generator=None, uniforms=No
     if not return_probs:
         res = accept(x, None, empty, temperature, u_resample=uniforms)
         return res.tokens[:, 0].long(), None
-    # tokens and probabilities from one draw (coopt_sample: the row statistics, then one
+    # tokens and probabilities from one draw (coopt_sample64: the row statistics, then one
     # launch that writes the probabilities and draws from them)
     lib = _lib.load()
     V = x.shape[1]
@@ -189,13 +189,13 @@ def sample(logits: torch.Tensor, temperature: float, generator=None, uniforms=No
     u = uniforms.to(device=x.device, dtype=torch.float32).contiguous()
     if u.numel() < N:
         raise ValueError("uniforms must have one entry per row")
-    tokens = torch.empty(N, dtype=torch.int32, device=x.device)
+    tokens = torch.empty(N, dtype=torch.int64, device=x.device)
     probs = torch.empty(x.shape, dtype=torch.float32, device=x.device)
-    _lib.check(lib.coopt_sample(_lib.dt_code(x.dtype), _lib.ptr(x), x.stride(0), N, V,
+    _lib.check(lib.coopt_sample64(_lib.dt_code(x.dtype), _lib.ptr(x), x.stride(0), N, V,
                                 float(temperature), _lib.ptr(u), _lib.ptr(tokens), None,
                                 _lib.ptr(probs), V, _lib.ptr(ws), ws.numel() * ws.element_size(),
-                                _lib.stream_handle(x.device)), "coopt_sample")
-    return tokens.long(), probs
+                                _lib.stream_handle(x.device)), "coopt_sample64")
+    return tokens, probs
 
 
 def verify(target_logits: torch.Tensor, draft_tokens, draft_probs, temperature: float,

@@ -392,6 +392,13 @@ int coopt_sample(int logits_dtype, const void* logits, int64_t row_stride, int N
                  float* probs, int64_t probs_stride, void* workspace, size_t workspace_bytes,
                  coopt_stream_t stream);
 
+/* coopt_sample with 64-bit tokens, the token type of sample()'s callers: the draw writes them
+ * itself, and no conversion launch follows. */
+int coopt_sample64(int logits_dtype, const void* logits, int64_t row_stride, int N, int V,
+                   float temperature, const float* uniforms, int64_t* tokens, float* margin,
+                   float* probs, int64_t probs_stride, void* workspace, size_t workspace_bytes,
+                   coopt_stream_t stream);
+
 /*
  * Elementwise stages of the Llama forward around the verify path (the model the step
  * benchmark runs), fused as the reference's forward fuses them (engine/model.py:234-254).

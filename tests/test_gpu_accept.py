@@ -327,3 +327,24 @@ def test_verify_signature_with_generator(dev):
     q = torch.softmax(torch.randn(2, V, generator=gen, device=dev), -1)
     out = M.verify(tl, [1, 2], q, 1.0, generator=gen)
     assert 1 <= len(out) <= 3 and all(0 <= t < V for t in out)
+
+
+@pytest.mark.parametrize("N,V,bf16", [(1, 5, False), (3, 8193, True), (33, 50257, False)])
+def test_sample64_draws_coopt_samples_tokens(dev, N, V, bf16):
+    """coopt_sample64 differs from coopt_sample in the type it stores a token in, nothing else."""
+    g = torch.Generator(device=dev).manual_seed(N + V)
+    x = (torch.randn(N, V, generator=g, device=dev) * 2).to(torch.bfloat16 if bf16 else torch.float32)
+    u = torch.rand(N, generator=g, device=dev)
+    L = M._lib.load()
+    ws = torch.empty(int(L.coopt_accept_sample_workspace(N, 0, V)), dtype=torch.uint8, device=dev)
+    got = []
+    for fn, dtype in ((L.coopt_sample, torch.int32), (L.coopt_sample64, torch.int64)):
+        tok = torch.full((N + 2,), -7, dtype=dtype, device=dev)
+        probs = torch.empty(N, V, device=dev)
+        M._lib.check(fn(M._lib.dt_code(x.dtype), M._lib.ptr(x), V, N, V, 0.9, M._lib.ptr(u), M._lib.ptr(tok), None,
+                      M._lib.ptr(probs), V, M._lib.ptr(ws), ws.numel(), M._lib.stream_handle(dev)), "sample")
+        assert (tok[N:] == -7).all()
+        got.append((tok[:N].long(), probs))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+    tok, probs = M.sample(x, 0.9, uniforms=u)
+    assert tok.dtype == torch.int64 and torch.equal(tok, got[0][0]) and torch.equal(probs, got[0][1])
