@@ -136,9 +136,17 @@ def runtime_version() -> int:
     return v.value
 
 
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def stream_handle(device=None) -> int:
-    """hipStream_t of torch's current stream on `device` (the stream every call uses)."""
-    return torch.cuda.current_stream(device).cuda_stream
+    """hipStream_t of torch's current stream on `device` (the stream every call uses).  By the
+    raw handle where torch has it: 0.1 us against 1.9 us for the Stream object, and a small
+    call's time is its host time (two handles a call with a workspace)."""
+    index = getattr(device, "index", device)
+    if _raw_stream is None or not (index is None or isinstance(index, int)):
+        return torch.cuda.current_stream(device).cuda_stream
+    return _raw_stream(torch.cuda.current_device() if index is None else index)
 
 
 def ptr(t) -> int:
@@ -173,8 +181,8 @@ class WorkspaceCache:
         self._retired = []
 
     def get(self, nbytes: int, device) -> torch.Tensor:
-        dev = torch.device(device)
-        key = (dev.index, torch.cuda.current_stream(dev).cuda_stream)
+        dev = device if isinstance(device, torch.device) else torch.device(device)
+        key = (dev.index, stream_handle(dev))
         buf = self._bufs.get(key)
         if buf is None or buf.numel() < nbytes:
             if buf is not None:

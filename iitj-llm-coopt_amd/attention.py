@@ -16,6 +16,7 @@ prefill chunks engine/engine.py:414-420 mixes into the same batch) run in query 
 64/(Hq/Hkv) rows, one block per window and KV head -- or, for long chunks, of 128/(Hq/Hkv) rows in a
 kernel that stages K and V in LDS for the window's rows.
 """
+import functools
 import math
 
 import torch
@@ -28,6 +29,7 @@ __all__ = ["flash_attn_varlen_func", "paged_attention", "paged_attention_qkv",
 _WS = _lib.WorkspaceCache()
 
 
+@functools.lru_cache(maxsize=1024)   # a pure function of the sizes; 0.9 us through ctypes
 def workspace_bytes(batch: int, num_heads: int, num_kv_heads: int, head_dim: int,
                     max_seqlen_q: int, max_seqlen_k: int) -> int:
     return int(_lib.load().coopt_verify_attention_workspace(batch, num_heads, num_kv_heads,

@@ -15,6 +15,7 @@ sample()/verify() are called with a torch.Generator instead, the uniforms are dr
 the output distribution is the target's (the rejection sampler is lossless), but the exact
 tokens differ from the reference's torch.multinomial stream.
 """
+import functools
 from dataclasses import dataclass
 
 import torch
@@ -37,6 +38,18 @@ class AcceptResult:
         acc = self.accepted_len.tolist()
         toks = self.tokens.tolist()
         return [row[: k + 1] for row, k in zip(toks, acc)]
+
+
+@functools.lru_cache(maxsize=1024)   # a pure function of the sizes; 0.9 us through ctypes
+def _workspace_bytes(batch, gamma_max, vocab):
+    return int(_lib.load().coopt_accept_sample_workspace(batch, gamma_max, vocab))
+
+
+def _on(x, dev, dtype):
+    """x on `dev` as contiguous `dtype` (x itself where it is that already)."""
+    if x.dtype == dtype and x.device == dev and x.is_contiguous():
+        return x
+    return x.to(device=dev, dtype=dtype).contiguous()
 
 
 def _rows(x):
@@ -69,7 +82,7 @@ def accept(target_logits, draft, draft_tokens, temperature, u_accept=None, u_res
     if tgt.dtype not in (torch.float32, torch.bfloat16):
         raise ValueError("target logits must be fp32 or bf16")
     V = tgt.shape[1]
-    dtok = draft_tokens.to(device=dev, dtype=torch.int32).contiguous()
+    dtok = _on(draft_tokens, dev, torch.int32)
     if dtok.dim() != 2:
         raise ValueError("draft_tokens must be [B, gamma_max]")
     B, gmax = dtok.shape
@@ -90,8 +103,8 @@ def accept(target_logits, draft, draft_tokens, temperature, u_accept=None, u_res
     if not greedy:
         if u_resample is None or (gmax > 0 and u_accept is None):
             raise ValueError("sampling needs u_accept [B, gamma_max] and u_resample [B]")
-    ua = None if u_accept is None else u_accept.to(device=dev, dtype=torch.float32).contiguous()
-    ur = None if u_resample is None else u_resample.to(device=dev, dtype=torch.float32).contiguous()
+    ua = None if u_accept is None else _on(u_accept, dev, torch.float32)
+    ur = None if u_resample is None else _on(u_resample, dev, torch.float32)
     if ua is not None and ua.numel() < B * gmax:
         raise ValueError("u_accept must have B*gamma_max entries")
     if ur is not None and ur.numel() < B:
@@ -131,7 +144,7 @@ def accept(target_logits, draft, draft_tokens, temperature, u_accept=None, u_res
             B, gmax, V, _lib.ptr(out.accepted_len), _lib.ptr(out.tokens), _lib.ptr(out.margin),
             _lib.stream_handle(dev)), "coopt_accept_sample_noalloc")
         return out
-    need = int(lib.coopt_accept_sample_workspace(B, gmax, V))
+    need = _workspace_bytes(B, gmax, V)
     if workspace is None:
         ws = _WS.get(need, dev)
     elif workspace.numel() * workspace.element_size() < need:
@@ -171,7 +184,8 @@ def sample(logits: torch.Tensor, temperature: float, generator=None, uniforms=No
     x, _ = _rows(logits)
     _lib.require_cuda(x)
     N = x.shape[0]
-    empty = torch.empty((N, 0), dtype=torch.int32, device=x.device)
+    if temperature <= 0 or not return_probs:
+        empty = torch.empty((N, 0), dtype=torch.int32, device=x.device)
     if temperature <= 0:
         res = accept(x, None, empty, 0.0)
         return res.tokens[:, 0].long(), None
@@ -184,9 +198,9 @@ def sample(logits: torch.Tensor, temperature: float, generator=None, uniforms=No
     # launch that writes the probabilities and draws from them)
     lib = _lib.load()
     V = x.shape[1]
-    need = int(lib.coopt_accept_sample_workspace(N, 0, V))
+    need = _workspace_bytes(N, 0, V)
     ws = _WS.get(need, x.device)
-    u = uniforms.to(device=x.device, dtype=torch.float32).contiguous()
+    u = _on(uniforms, x.device, torch.float32)
     if u.numel() < N:
         raise ValueError("uniforms must have one entry per row")
     tokens = torch.empty(N, dtype=torch.int64, device=x.device)
