@@ -247,6 +247,34 @@ def test_linear_silu_is_bit_identical_to_linear_then_silu(dev, M, F, K):
     assert torch.equal(got.view(torch.int16), want.view(torch.int16))
 
 
+@pytest.mark.parametrize("M,off,ld", [(32, 1, 519), (17, 2, 514), (64, 3, 517)])
+def test_linear_silu_writes_rows_at_any_element(dev, M, off, ld):
+    """Output rows may start at any element and lie any number of elements apart."""
+    F, K = 512, 256
+    g = torch.Generator(device=dev).manual_seed(M)
+    x = torch.randn(M, K, generator=g, device=dev).to(torch.bfloat16)
+    w = fused.pack_gate_up_weight((torch.randn(2 * F, K, generator=g, device=dev) * 0.05).to(torch.bfloat16))
+    store = torch.full((off + M * ld,), 7.0, dtype=torch.bfloat16, device=dev)
+    rows = store[off:].view(M, ld)
+    fused.linear_silu(x, w, out=rows[:, :F])
+    assert torch.equal(rows[:, :F], fused.linear_silu(x, w))
+    assert (rows[:, F:] == 7).all() and (store[:off] == 7).all()
+
+
+@pytest.mark.parametrize("M,off,ld", [(32, 1, 519), (17, 2, 514), (64, 3, 517)])
+def test_linear_silu_writes_rows_at_any_element(dev, M, off, ld):
+    """Output rows may start at any element and lie any number of elements apart."""
+    F, K = 512, 256
+    g = torch.Generator(device=dev).manual_seed(M)
+    x = torch.randn(M, K, generator=g, device=dev).to(torch.bfloat16)
+    w = fused.pack_gate_up_weight((torch.randn(2 * F, K, generator=g, device=dev) * 0.05).to(torch.bfloat16))
+    store = torch.full((off + M * ld,), 7.0, dtype=torch.bfloat16, device=dev)
+    rows = store[off:].view(M, ld)
+    fused.linear_silu(x, w, out=rows[:, :F])
+    assert torch.equal(rows[:, :F], fused.linear_silu(x, w))
+    assert (rows[:, F:] == 7).all() and (store[:off] == 7).all()
+
+
 def test_linear_silu_falls_back_outside_the_fused_shapes(dev):
     """160 rows (a split K and 8 waves) and torch-sized row counts take the two-step path."""
     g = torch.Generator(device=dev).manual_seed(2)
