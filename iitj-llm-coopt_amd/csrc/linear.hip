@@ -11,13 +11,13 @@
 // Decomposition.  A workgroup of WAVES waves owns WAVES * NW 16-column tiles of the output
 // and a K range of `kt` elements; gridDim.y workgroups split K, and when it exceeds one they
 // write fp32 partials that reduce_kernel sums in a fixed order (deterministic, no atomics).
-//   * W streams from HBM straight into MFMA A operands: per 128-wide K step a lane reads 64
+//   * W streams from HBM straight into MFMA B operands: per 128-wide K step a lane reads 64
 //     contiguous bytes of its output row as 4 x 16 B (MFMA j covers k0 + 32j + [8g, 8g+8),
 //     g = lane / 16), PF steps ahead of the MFMAs.
 //   * X is shared: each K step's [M, 128] slice is staged once per workgroup in LDS (double
-//     buffered, rows padded to 288 bytes) and read by all waves as MFMA B operands.
-//   * v_mfma_f32_16x16x32_bf16 with A = W rows, B = X rows: lane l holds
-//     C^T[4(l/16) + i][l % 16] of each 16x16 tile, four consecutive columns of one row.
+//     buffered, rows padded to 288 bytes) and read by all waves as MFMA A operands.
+//   * v_mfma_f32_16x16x32_bf16 with A = X rows, B = W rows: lane l holds
+//     C[4(l/16) + i][l % 16] of each 16x16 tile (SILU: A = W, B = X, the transpose).
 //
 // Tile-packed weights (coopt_linear_pack_weight).  W may instead be stored as [N/16][K/128]
 // tiles of 16 rows x 128 K, each the 4 x 64 16-byte chunks in the order the lanes load them:
@@ -32,6 +32,9 @@ namespace {
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
+// four bf16 of a row that need not start at a multiple of 8 bytes
+typedef uint32_t u32x2_any_t __attribute__((ext_vector_type(2), aligned(2)));
 
 constexpr int kKB = 128;                  // K elements per step
 // LDS bytes per staged X row.  A fragment read has 16 lanes at consecutive rows and four 16-byte
@@ -162,7 +165,8 @@ __global__ __launch_bounds__(64 * WAVES) void linear_kernel(
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-      for (int nt = 0; nt < NW; ++nt) acc[mt][nt] = mfma_bf16(wr[nt][j], fa[mt], acc[mt][nt]);
+      for (int nt = 0; nt < NW; ++nt)
+        acc[mt][nt] = SILU ? mfma_bf16(wr[nt][j], fa[mt], acc[mt][nt]) : mfma_bf16(fa[mt], wr[nt][j], acc[mt][nt]);
   };
   // (sched_barrier keeps the scheduler from sinking the reads back next to their MFMAs)
   auto compute = [&](int buf, const u32x4_t (&wr)[NW][4]) {
@@ -208,14 +212,8 @@ __global__ __launch_bounds__(64 * WAVES) void linear_kernel(
     }
   }
 
-  // Epilogue.  W is the MFMAs' A operand and X their B, so a lane holds four consecutive
-  // columns, n0 + 16 nt + 4 g + i, of row 16 mt + l16: one 16-byte (bf16: 8-byte) store per tile
-  // instead of four of one column each.
-  auto pack4 = [](const f32x4_t& v) {
-    return make_uint2(f32_to_bf16(v[0]) | (static_cast<uint32_t>(f32_to_bf16(v[1])) << 16),
-                      f32_to_bf16(v[2]) | (static_cast<uint32_t>(f32_to_bf16(v[3])) << 16));
-  };
   if constexpr (SILU) {
+    // W is the A operand: a lane holds four consecutive outputs of a row for its 8-byte stores.
     // Wave 2p holds gate tile t = blockIdx.x * WAVES / 2 + p and wave 2p + 1 the matching up
     // tile.  They hand each other half of their row tiles through LDS (the X staging is dead by
     // now) and finish the other half each.  Each sum is rounded to bf16 first -- the
@@ -227,6 +225,10 @@ __global__ __launch_bounds__(64 * WAVES) void linear_kernel(
     f32x4_t* xch = reinterpret_cast<f32x4_t*>(&xs[0][0]) + (wave >> 1) * (MT * 64) + lane;
     const int F = a.N / 2;
     const int j = (blockIdx.x * (WAVES / 2) + (wave >> 1)) * 16 + 4 * g;
+    auto pack4 = [](const f32x4_t& v) {
+      return u32x2_t{f32_to_bf16(v[0]) | (static_cast<uint32_t>(f32_to_bf16(v[1])) << 16),
+                     f32_to_bf16(v[2]) | (static_cast<uint32_t>(f32_to_bf16(v[3])) << 16)};
+    };
     auto finish = [&](int mt, const f32x4_t& gate, const f32x4_t& up) {
       const int m = mt * 16 + l16;
       f32x4_t r;
@@ -237,7 +239,7 @@ __global__ __launch_bounds__(64 * WAVES) void linear_kernel(
         r[i] = gv / (1.0f + __expf(-gv)) * uv;
       }
       if (m < a.M && j < F)
-        *reinterpret_cast<uint2*>(a.y + static_cast<int64_t>(m) * a.ldy + j) = pack4(r);
+        *reinterpret_cast<u32x2_any_t*>(a.y + static_cast<int64_t>(m) * a.ldy + j) = pack4(r);
     };
     if (wave & 1) {
 #pragma unroll
@@ -254,27 +256,36 @@ __global__ __launch_bounds__(64 * WAVES) void linear_kernel(
     }
     return;
   }
+  // Epilogue: X is the MFMAs' A operand, so a lane holds rows 16 mt + 4 g + i of column
+  // n0 + 16 nt + l16, and 16 lanes store 64 (bf16: 32) contiguous bytes of one row at once.  With W as
+  // A a lane has four columns of one row: one store instead of four, but 16 lanes then touch 16
+  // rows, and the partials of 65 to 96 rows cost 1.5 us more (90 x 3072 x 2048 9.0 -> 9.9 us, 80 x
+  // 6144 x 4096 15.7 -> 17.2; draft forwards of 192, 160 and 90 rows, two layers and logits: 385 / 347 /
+  // 303 us with W as A, 367 / 339 / 296 like this).
   if (gridDim.y == 1 && !a.force_part) {
 #pragma unroll
     for (int nt = 0; nt < NW; ++nt) {
-      const int n = n0 + nt * 16 + 4 * g;
+      const int n = n0 + nt * 16 + l16;
       if (n >= a.N) continue;
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt) {
-        const int m = mt * 16 + l16;
-        if (m < a.M)
-          *reinterpret_cast<uint2*>(a.y + static_cast<int64_t>(m) * a.ldy + n) = pack4(acc[mt][nt]);
-      }
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int m = mt * 16 + 4 * g + i;
+          if (m < a.M) a.y[static_cast<int64_t>(m) * a.ldy + n] = f32_to_bf16(acc[mt][nt][i]);
+        }
     }
   } else {
     float* p = a.part + static_cast<int64_t>(blockIdx.y) * (MT * 16) * a.N;
 #pragma unroll
     for (int nt = 0; nt < NW; ++nt) {
-      const int n = n0 + nt * 16 + 4 * g;
+      const int n = n0 + nt * 16 + l16;
       if (n >= a.N) continue;
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt)
-        *reinterpret_cast<f32x4_t*>(p + static_cast<int64_t>(mt * 16 + l16) * a.N + n) = acc[mt][nt];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          p[static_cast<int64_t>(mt * 16 + 4 * g + i) * a.N + n] = acc[mt][nt][i];
     }
   }
 }
