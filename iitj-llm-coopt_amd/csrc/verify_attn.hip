@@ -1124,7 +1124,8 @@ __global__ __launch_bounds__(kThreads) void merge_kernel(AttnArgs a) {
 // and 32 rows) and, where windows are few, its chain per stage (1.3-2 us: staging 1.0 without the
 // tiles' work, the tiles 0.5-1.0).  Chunks of 1500 and 500 rows with 16 verify items of 5 rows
 // (bf16, 32/8 heads of 128, 30 GFLOP): 138 us on verify_attn_kernel's windows of 64 rows, whose
-// waves each read their own keys, 69 us here; INT8 190 and 82.
+// waves each read their own keys, 66 us here; INT8 190 and 82.  (l as a product of the rounded
+// probabilities with ones: 67.4 us, and no longer a sum of 32-bit probabilities.)
 // Tried: 64 keys per softmax (66-72 us, but 50 instead of 42 us for 2000 keys of a verify item alone,
 // which two waves share below), one stage of loads in flight with an L2 touch ahead (72).
 // Blocks take the windows with most keys first: window r from the end of every sequence before
@@ -1401,9 +1402,10 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(AttnArgs a) {
       }
     }
     // bf16 probabilities: the reference is the running maximum itself (no slack), so the largest
-    // one is exactly 1; with the slack and unrounded sums one reference for all keys was 2 %
-    // further from 64 bits than verify_attn_kernel's one per wave (2.10e-3 against 2.05e-3 relative
-    // in the batch above; like this 2.01e-3)
+    // one is exactly 1; with the slack one reference for all keys was 2 % further from 64 bits than
+    // verify_attn_kernel's one per wave (2.10e-3 against 2.05e-3 relative in the batch above; like
+    // this 2.02e-3; the largest excess over seven batches, 600 + 100 rows and 2 items: 1.977e-3
+    // against 1.968e-3)
     constexpr float kSlack = INT8 ? 8.0f : 0.0f;
     if (kb + 31 > first_lim) {  // some row does not see every key (those past L are past it)
 #pragma unroll
@@ -1447,8 +1449,8 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(AttnArgs a) {
         float pr[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) pr[i] = exp2_fast(fmaf(acc[rt][kt][i], a.scale_log2, -m_use));
+        l_run[rt] += (pr[0] + pr[1]) + (pr[2] + pr[3]);
         if constexpr (INT8) {
-          l_run[rt] += (pr[0] + pr[1]) + (pr[2] + pr[3]);
 #pragma unroll
           for (int i = 0; i < 4; ++i)
             pr[i] *= f16_to_f32(static_cast<uint16_t>(vs[kt][i >> 1] >> (16 * (i & 1))));
@@ -1459,19 +1461,6 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(AttnArgs a) {
           pb[rt][kt >> 1][2 * (kt & 1)] = p0;
           pb[rt][kt >> 1][2 * (kt & 1) + 1] = p1;
         }
-      }
-    }
-    if constexpr (!INT8) {
-      // l: the sum of the rounded probabilities (their common rounding cancels in o / l), as a
-      // product with ones
-      constexpr uint32_t kOnes = 0x3f803f80u;
-      const u32x4_t ones = {kOnes, kOnes, kOnes, kOnes};
-#pragma unroll
-      for (int rt = 0; rt < 2; ++rt) {
-        f32x4_t sum = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int t = 0; t < kSub / 2; ++t) sum = mfma_bf16(ones, pb[rt][t], sum);
-        l_run[rt] += sum[0];
       }
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -1523,13 +1512,10 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(AttnArgs a) {
       compute(s + 1);
     }
   }
-  // bf16: every lane of a row's column holds its whole sum already
-  if constexpr (INT8) {
 #pragma unroll
-    for (int rt = 0; rt < 2; ++rt) {
-      l_run[rt] = add_xor32(add_xor16(l_run[rt]));
-      m_run[rt] += static_cast<float>(e_v);  // o and l are relative to 2^(m_run + e_v)
-    }
+  for (int rt = 0; rt < 2; ++rt) {
+    l_run[rt] = add_xor32(add_xor16(l_run[rt]));
+    if constexpr (INT8) m_run[rt] += static_cast<float>(e_v);  // o and l are relative to 2^(m_run + e_v)
   }
   if (pair) {  // waves 2 and 3 hand their sums to waves 0 and 1
     constexpr int kWords = 2 * kDt + 1;
