@@ -144,7 +144,8 @@ def stream_handle(device=None) -> int:
     raw handle where torch has it: 0.1 us against 1.9 us for the Stream object, and a small
     call's time is its host time (two handles a call with a workspace)."""
     index = getattr(device, "index", device)
-    if _raw_stream is None or not (index is None or isinstance(index, int)):
+    if (_raw_stream is None or not (index is None or isinstance(index, int))
+            or getattr(device, "type", "cuda") != "cuda"):   # torch refuses other devices
         return torch.cuda.current_stream(device).cuda_stream
     return _raw_stream(torch.cuda.current_device() if index is None else index)
 

@@ -206,9 +206,9 @@ def sample(logits: torch.Tensor, temperature: float, generator=None, uniforms=No
     tokens = torch.empty(N, dtype=torch.int64, device=x.device)
     probs = torch.empty(x.shape, dtype=torch.float32, device=x.device)
     _lib.check(lib.coopt_sample64(_lib.dt_code(x.dtype), _lib.ptr(x), x.stride(0), N, V,
-                                float(temperature), _lib.ptr(u), _lib.ptr(tokens), None,
-                                _lib.ptr(probs), V, _lib.ptr(ws), ws.numel() * ws.element_size(),
-                                _lib.stream_handle(x.device)), "coopt_sample64")
+                                  float(temperature), _lib.ptr(u), _lib.ptr(tokens), None,
+                                  _lib.ptr(probs), V, _lib.ptr(ws), ws.numel() * ws.element_size(),
+                                  _lib.stream_handle(x.device)), "coopt_sample64")
     return tokens, probs
 
 
