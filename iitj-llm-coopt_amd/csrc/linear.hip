@@ -241,16 +241,21 @@ __global__ __launch_bounds__(64 * WAVES) void linear_kernel(
       if (m < a.M && j < F)
         *reinterpret_cast<u32x2_any_t*>(a.y + static_cast<int64_t>(m) * a.ldy + j) = pack4(r);
     };
-    if (wave & 1) {
+    // The wave's role in a scalar register and one barrier for both waves of a pair: a barrier inside the
+    // arms of a branch on threadIdx would rest on each wave skipping the other's arm.
+    const bool up_wave = __builtin_amdgcn_readfirstlane(wave) & 1;
+    if (up_wave) {
 #pragma unroll
       for (int mt = 0; mt < kHalf; ++mt) xch[mt * 64] = acc[mt][0];
-      __syncthreads();
-#pragma unroll
-      for (int mt = kHalf; mt < MT; ++mt) finish(mt, xch[mt * 64], acc[mt][0]);
     } else {
 #pragma unroll
       for (int mt = kHalf; mt < MT; ++mt) xch[mt * 64] = acc[mt][0];
-      __syncthreads();
+    }
+    __syncthreads();
+    if (up_wave) {
+#pragma unroll
+      for (int mt = kHalf; mt < MT; ++mt) finish(mt, xch[mt * 64], acc[mt][0]);
+    } else {
 #pragma unroll
       for (int mt = 0; mt < kHalf; ++mt) finish(mt, acc[mt][0], xch[mt * 64]);
     }

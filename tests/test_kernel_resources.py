@@ -43,3 +43,30 @@ def test_no_kernel_spills_to_scratch(tmp_path):
     assert len(kernels) > 20, kernels  # the report was parsed
     spilled = {k: v for k, v in kernels.items() if v}
     assert not spilled, f"kernels using scratch (bytes/lane): {spilled}"
+
+
+@pytest.mark.skipif(HIPCC is None, reason="hipcc not installed")
+def test_projection_barriers_are_reached_by_every_wave(tmp_path):
+    """The projection kernels' waves branch on their index before the last barrier (the fused
+    SiLU's exchange): no execution mask is narrowed up to there, so no barrier lies in an arm
+    that a wave might skip or pass through with its lanes off."""
+    resources("linear.hip", str(tmp_path))
+    kernels, name = {}, None
+    for line in open(os.path.join(str(tmp_path), "linear.hip.s")):
+        m = re.match(r"(_Z\w*linear_kernel\w*):", line)
+        if m:
+            name = m.group(1)
+            kernels[name] = []
+        elif line.startswith(".Lfunc_end"):
+            name = None
+        elif name:
+            kernels[name].append(line.split(";")[0])
+    assert len(kernels) > 20, list(kernels)
+    narrowed = re.compile(r"_saveexec_b64|s_\w+_b64 exec,|v_cmpx_")
+    bad = {}
+    for k, lines in kernels.items():
+        last = max(i for i, line in enumerate(lines) if "s_barrier" in line)
+        hits = [line.strip() for line in lines[:last] if narrowed.search(line)]
+        if hits:
+            bad[k] = hits[:3]
+    assert not bad, bad
