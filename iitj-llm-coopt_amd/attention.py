@@ -13,8 +13,8 @@ pass k_scale/v_scale; dequantisation is fused into the kernel.
 Supported: head_dim 64 or 128, any q_len.  Items of up to 64 rows per KV head, (Hq/Hkv) *
 max_seqlen_q <= 64 (speculative verify and decode), take the tuned path; longer ones (the
 prefill chunks engine/engine.py:414-420 mixes into the same batch) run in query windows of
-64/(Hq/Hkv) rows, one block per window and KV head -- or, for long chunks, of 128/(Hq/Hkv) rows in a
-kernel that stages K and V in LDS for the window's rows.
+64/(Hq/Hkv) rows, one block per window and KV head -- or, where the batch has windows enough to fill
+the GPU, of 128/(Hq/Hkv) rows in a kernel that stages K and V in LDS for the window's rows.
 """
 import functools
 import math
@@ -89,11 +89,11 @@ def paged_attention(q, k_cache, v_cache, cu_seqlens_q, seq_lens, block_table, ma
         raise ValueError(f"workspace holds {workspace.numel() * workspace.element_size()} "
                          f"bytes, {need} needed")
     cs = k_cache.stride()
-    _lib.check(lib.coopt_verify_attention(
+    _lib.check(lib.coopt_verify_attention_rows(
         code, _lib.ptr(q), q.stride(0), q.stride(1), _lib.ptr(k_cache), _lib.ptr(v_cache),
         cs[0], cs[1], cs[2], _lib.ptr(ks), _lib.ptr(vs), sstr[0], sstr[1], sstr[2],
         _lib.ptr(block_table), block_table.stride(0), _lib.ptr(cu), _lib.ptr(sl),
-        B, Hq, Hkv, D, bs, NB, int(max_seqlen_q), int(max_seqlen_k), float(softmax_scale),
+        B, Hq, Hkv, D, bs, NB, int(max_seqlen_q), int(max_seqlen_k), T, float(softmax_scale),
         _lib.ptr(out), out.stride(0), out.stride(1), _lib.ptr(workspace),
         workspace.numel() * workspace.element_size(), _lib.stream_handle(q.device)),
         "coopt_verify_attention")

@@ -1600,21 +1600,67 @@ struct AttnShape {
 };
 
 constexpr int kMaxRows = 64;
-// Which of the two takes a windowed call.  prefill_attn_kernel has the higher rate,
-// verify_attn_kernel the shorter chain per window (its four waves share a window's keys), so the
-// first takes calls that may hold many windows: chunks of 2048 rows (512 tokens at G = 4) or
-// more, or 32 sequences with items of 256 rows.  bf16, 32/8 heads of 128, old / new us: chunks of
-// 1500 + 500 rows and 16 verify items 138 / 69, 512 + 17 and 20 66 / 27, 2048 + 1000 and 32 388 / 182,
-// 600 + 100 and 2 65 / 68, 64 + 17 and 32 109 / 60; below the line 300 + 100 and 8 70 / 80, 260 + 17 and
-// 2 52 / 66, 17 + 17 and 4 35 / 64.
-constexpr int kPrefillFrom = 2048, kPrefillFromMany = 256, kManySeqs = 32;
+// Which of the two takes a windowed call.  verify_attn_kernel has the shorter chain per window (its
+// four waves share the window's keys: a window of 4096 keys takes it 60 us, 119 in prefill_attn_kernel),
+// prefill_attn_kernel the higher rate once the GPU is full.  Estimated from the window counts, in us:
+//   verify_attn_kernel   8 + 0.0135 k (INT8 0.0185 k) per round of 256 windows over k keys, 5 ns per
+//                        block of the grid without rows.  Blocks go to the 32 pairs of XCD and
+//                        shader engine in turn, so where the sequences' first windows lie a
+//                        multiple apart in the grid, the items of one window share a part of the pairs
+//                        (a chunk of 64 tokens with 16 items of 5, 4096 keys: 182 us, of 33 tokens: 67)
+//   prefill_attn_kernel  6.5 + 0.038 k per round of 512 windows (two on a CU), by halves; 1.4 ns per
+//                        block without rows; it packs its windows unless B > kPlanSeqs
+// Fitted to 2784 batches of 1 to 70 sequences, chunks of 17 to 2100 tokens, 17 to 18000 keys, 1 to 16 KV
+// heads, G 1 to 8, bf16 and INT8, head dims 64 and 128: against verify_attn_kernel for all of them the
+// times' mean is 0.77 (the faster kernel each time: 0.76), 16 batches are more than 3 % slower, the
+// worst 1.18 (prefill_attn_kernel for all: 1.97).  us, verify / prefill, bf16, 32/8 heads of 128: a chunk of 512
+// tokens over 512 keys 14.8 / 21.1, over 16384 240 / 438, with 16 items of 5 over 16384 713 / 449; 1024
+// over 4096 114 / 120; 2048 over 4096 197 / 143; 16 chunks of 256 over 4096 504 / 347.
+bool prefill_is_faster(int B, int G, int Hkv, int max_seqlen_q, int max_seqlen_k, int64_t total_q, bool int8) {
+  constexpr double kCus = 256;
+  const int64_t others = total_q > max_seqlen_q ? total_q - max_seqlen_q : 0;  // rows of the other sequences
+  struct Grid {
+    double longest, rest;  // blocks of the longest item; of the others, one window each at least
+    double firsts;         // of the others' first windows alone
+    double empty;          // without rows
+    double pairs;          // share of the pairs that the first windows fall on
+  };
+  auto grid = [&](int rows) {
+    const int64_t qwin = rows / G, per_seq = (max_seqlen_q + qwin - 1) / qwin;
+    Grid g;
+    g.longest = static_cast<double>(per_seq) * Hkv;
+    g.firsts = static_cast<double>(B - 1) * Hkv;
+    g.rest = fmax(g.firsts, B > 1 ? static_cast<double>((others + qwin - 1) / qwin) * Hkv : 0.0);
+    g.empty = fmax(0.0, g.longest * B - g.longest - g.rest);
+    int64_t apart = per_seq * Hkv % 32, step = 32;  // step: the greatest common divisor with 32
+    while (apart) {
+      const int64_t t = step % apart;
+      step = apart;
+      apart = t;
+    }
+    g.pairs = fmin(1.0, static_cast<double>(Hkv) / static_cast<double>(step));
+    return g;
+  };
+  const Grid v = grid(kMaxRows), p = grid(kPrefillRows);
+  // a chunk's earlier windows see fewer keys
+  const double k = max_seqlen_k, seen = 1.0 - 0.125 * fmin(1.0, max_seqlen_q / k);
+  double v_rounds = fmax(1.0, ceil((v.longest * seen + v.rest) / kCus));
+  double p_rounds = fmax(1.0, 0.5 * ceil((p.longest * seen + p.rest) / kCus));
+  if (B > 1) v_rounds = fmax(v_rounds, ceil(0.4 * v.longest / kCus + v.firsts / (kCus * v.pairs)));
+  if (B > kPlanSeqs) p_rounds = fmax(p_rounds, ceil(0.5 * p.firsts / (kCus * p.pairs)));
+  const double v_us = v_rounds * (8.0 + (int8 ? 0.0185 : 0.0135) * k) + 0.005 * v.empty;
+  const double p_us = p_rounds * (6.5 + 0.038 * k) + 0.0014 * p.empty;
+  return 1.03 * p_us < v_us;
+}
 
-AttnShape attn_shape(int B, int G, int Hkv, int max_seqlen_q, int max_seqlen_k) {
+// total_q: the call's query rows, 0 if unknown (one row for every sequence but the longest then);
+// it and int8 decide between the window kernels only, not any workspace.
+AttnShape attn_shape(int B, int G, int Hkv, int max_seqlen_q, int max_seqlen_k, int64_t total_q, bool int8) {
   AttnShape s{};
   if (G * static_cast<int64_t>(max_seqlen_q) > kMaxRows) {
     // longer items run in query windows of kMaxRows (verify_attn_kernel: a wave's tiles are its
     // own, which suits few windows) or kPrefillRows rows (prefill_attn_kernel)
-    s.prefill = G * static_cast<int64_t>(max_seqlen_q) >= (B >= kManySeqs ? kPrefillFromMany : kPrefillFrom);
+    s.prefill = prefill_is_faster(B, G, Hkv, max_seqlen_q, max_seqlen_k, total_q, int8);
     s.qwin = (s.prefill ? kPrefillRows : kMaxRows) / G;
     s.nwin = (max_seqlen_q + s.qwin - 1) / s.qwin;
     s.rmax = G * s.qwin;
@@ -1702,7 +1748,7 @@ extern "C" size_t coopt_verify_attention_workspace(int B, int Hq, int Hkv, int D
   if (B <= 0 || Hkv <= 0 || Hq <= 0 || Hq % Hkv || Hq / Hkv > kMaxRows || max_seqlen_q <= 0 ||
       max_seqlen_k <= 0)
     return 0;
-  const AttnShape sh = attn_shape(B, Hq / Hkv, Hkv, max_seqlen_q, max_seqlen_k);
+  const AttnShape sh = attn_shape(B, Hq / Hkv, Hkv, max_seqlen_q, max_seqlen_k, 0, false);
   if (sh.nwin > 0) return 256;  // one split per window: no partials
   return attn_ws_layout(B, Hkv, D, sh.rmax, sh.max_splits).total;
 }
@@ -1740,9 +1786,9 @@ int verify_attention_impl(const char* who, const FusedQkv* fz, int kv_dtype, con
                           const int32_t* block_table, int64_t bt_stride,
                           const int32_t* cu_seqlens_q, const int32_t* seq_lens, int B, int Hq,
                           int Hkv, int D, int block_size, int64_t num_blocks, int max_seqlen_q,
-                          int max_seqlen_k, float softmax_scale, void* out, int64_t o_tok_stride,
-                          int64_t o_head_stride, void* workspace, size_t workspace_bytes,
-                          coopt_stream_t stream) {
+                          int max_seqlen_k, int64_t total_q, float softmax_scale, void* out,
+                          int64_t o_tok_stride, int64_t o_head_stride, void* workspace,
+                          size_t workspace_bytes, coopt_stream_t stream) {
   ATTN_REQUIRE(kv_dtype == COOPT_DT_BF16 || kv_dtype == COOPT_DT_I8,
                "kv_dtype must be COOPT_DT_BF16 or COOPT_DT_I8");
   ATTN_REQUIRE(B >= 0 && Hq > 0 && Hkv > 0 && Hq % Hkv == 0, "Hq must be a multiple of Hkv");
@@ -1811,7 +1857,7 @@ int verify_attention_impl(const char* who, const FusedQkv* fz, int kv_dtype, con
   a.out = static_cast<uint16_t*>(out);
   a.o_ts = o_tok_stride;
   a.o_hs = o_head_stride;
-  const AttnShape shape = attn_shape(B, G, Hkv, max_seqlen_q, max_seqlen_k);
+  const AttnShape shape = attn_shape(B, G, Hkv, max_seqlen_q, max_seqlen_k, total_q, int8);
   // grid limits: 2^32 work-items along x, 65535 blocks along z
   ATTN_REQUIRE(shape.nwin == 0 || static_cast<int64_t>(B) * shape.nwin * Hkv < (int64_t{1} << 24),
                "too many query windows for one launch");
@@ -1896,8 +1942,41 @@ extern "C" int coopt_verify_attention(int kv_dtype, const void* q, int64_t q_tok
                                c_head_stride, k_scale, v_scale, s_blk_stride, s_tok_stride,
                                s_head_stride, block_table, bt_stride, cu_seqlens_q, seq_lens, B,
                                Hq, Hkv, D, block_size, num_blocks, max_seqlen_q, max_seqlen_k,
-                               softmax_scale, out, o_tok_stride, o_head_stride, workspace,
+                               0, softmax_scale, out, o_tok_stride, o_head_stride, workspace,
                                workspace_bytes, stream);
+}
+
+extern "C" int coopt_verify_attention_rows(int kv_dtype, const void* q, int64_t q_tok_stride,
+                                           int64_t q_head_stride, const void* k_cache,
+                                           const void* v_cache, int64_t c_blk_stride,
+                                           int64_t c_tok_stride, int64_t c_head_stride,
+                                           const void* k_scale, const void* v_scale,
+                                           int64_t s_blk_stride, int64_t s_tok_stride,
+                                           int64_t s_head_stride, const int32_t* block_table,
+                                           int64_t bt_stride, const int32_t* cu_seqlens_q,
+                                           const int32_t* seq_lens, int B, int Hq, int Hkv, int D,
+                                           int block_size, int64_t num_blocks, int max_seqlen_q,
+                                           int max_seqlen_k, int64_t total_q, float softmax_scale,
+                                           void* out,
+                                           int64_t o_tok_stride, int64_t o_head_stride,
+                                           void* workspace, size_t workspace_bytes,
+                                           coopt_stream_t stream) {
+  return verify_attention_impl("coopt_verify_attention", nullptr, kv_dtype, q, q_tok_stride,
+                               q_head_stride, k_cache, v_cache, c_blk_stride, c_tok_stride,
+                               c_head_stride, k_scale, v_scale, s_blk_stride, s_tok_stride,
+                               s_head_stride, block_table, bt_stride, cu_seqlens_q, seq_lens, B,
+                               Hq, Hkv, D, block_size, num_blocks, max_seqlen_q, max_seqlen_k,
+                               total_q, softmax_scale, out, o_tok_stride, o_head_stride, workspace,
+                               workspace_bytes, stream);
+}
+
+extern "C" int coopt_verify_attention_window_rows(int kv_dtype, int B, int Hq, int Hkv, int max_seqlen_q,
+                                                 int max_seqlen_k, int64_t total_q) {
+  if (B <= 0 || Hkv <= 0 || Hq <= 0 || Hq % Hkv || Hq / Hkv > kMaxRows || max_seqlen_q <= 0 ||
+      max_seqlen_k <= 0)
+    return 0;
+  const AttnShape s = attn_shape(B, Hq / Hkv, Hkv, max_seqlen_q, max_seqlen_k, total_q, kv_dtype == COOPT_DT_I8);
+  return s.nwin == 0 ? 0 : s.prefill ? kPrefillRows : kMaxRows;
 }
 
 extern "C" int coopt_verify_attention_qkv_supported(int kv_dtype, int B, int Hq, int Hkv, int D,
@@ -1908,7 +1987,7 @@ extern "C" int coopt_verify_attention_qkv_supported(int kv_dtype, int B, int Hq,
   const int G = Hq / Hkv;
   if (static_cast<int64_t>(G) * max_seqlen_q > kMaxRows) return 0;
   if (!fused_ok(D, kv_dtype == COOPT_DT_I8, (G * max_seqlen_q + 15) / 16)) return 0;
-  return attn_shape(B, G, Hkv, max_seqlen_q, max_seqlen_k).max_splits == 1 ? 1 : 0;
+  return attn_shape(B, G, Hkv, max_seqlen_q, max_seqlen_k, 0, false).max_splits == 1 ? 1 : 0;
 }
 
 extern "C" int coopt_verify_attention_qkv(
@@ -1927,7 +2006,7 @@ extern "C" int coopt_verify_attention_qkv(
                                k_cache, v_cache, c_blk_stride, c_tok_stride, c_head_stride,
                                k_scale, v_scale, s_blk_stride, s_tok_stride, s_head_stride,
                                block_table, bt_stride, cu_seqlens_q, seq_lens, B, Hq, Hkv, D,
-                               block_size, num_blocks, max_seqlen_q, max_seqlen_k, softmax_scale,
+                               block_size, num_blocks, max_seqlen_q, max_seqlen_k, 0, softmax_scale,
                                out, o_tok_stride, o_head_stride, workspace, workspace_bytes,
                                stream);
 }

@@ -243,9 +243,11 @@ int coopt_kv_copy_blocks(const int64_t* regions, int num_regions, const int64_t*
  *   (speculative verify and decode), run on the tuned path (contexts split over blocks).
  *   Longer items -- the prefill chunks the engine mixes into one batch with its verify items
  *   (engine/engine.py:414-420), or a long draft catch-up -- run in query windows, each one
- *   block over the keys its last row sees: of 64/(Hq/Hkv) rows, or, with chunks of 2048 rows
- *   per KV head (or 256 in batches of 32 sequences) and more, of 128/(Hq/Hkv) rows in a kernel
- *   that stages K and V in LDS (B * windows * Hkv < 2^24 blocks).
+ *   block over the keys its last row sees: of 64/(Hq/Hkv) rows, or, where the batch's windows
+ *   fill the GPU well enough for it to be the faster one, of 128/(Hq/Hkv) rows in a kernel that
+ *   stages K and V in LDS (B * windows * Hkv < 2^24 blocks).  That choice needs the call's
+ *   query rows: coopt_verify_attention_rows takes them, coopt_verify_attention assumes one
+ *   row for every sequence but the longest.
  *   Callers must keep seq_lens <= max_seqlen_k, q rows per sequence
  *   <= max_seqlen_q and block ids in [0, num_blocks); the kernel clamps all three so a
  *   malformed call yields wrong rows but never an access outside its buffers.
@@ -268,6 +270,25 @@ int coopt_verify_attention(int kv_dtype,
                            int max_seqlen_q, int max_seqlen_k, float softmax_scale,
                            void* out, int64_t o_tok_stride, int64_t o_head_stride,
                            void* workspace, size_t workspace_bytes, coopt_stream_t stream);
+/* coopt_verify_attention, told the query rows of the call (q's first dimension; 0: unknown).
+ * They decide how items of more than 64 rows per KV head are cut into windows, nothing else. */
+int coopt_verify_attention_rows(int kv_dtype,
+                                const void* q, int64_t q_tok_stride, int64_t q_head_stride,
+                                const void* k_cache, const void* v_cache,
+                                int64_t c_blk_stride, int64_t c_tok_stride, int64_t c_head_stride,
+                                const void* k_scale, const void* v_scale,
+                                int64_t s_blk_stride, int64_t s_tok_stride, int64_t s_head_stride,
+                                const int32_t* block_table, int64_t bt_stride,
+                                const int32_t* cu_seqlens_q, const int32_t* seq_lens,
+                                int B, int Hq, int Hkv, int D, int block_size, int64_t num_blocks,
+                                int max_seqlen_q, int max_seqlen_k, int64_t total_q,
+                                float softmax_scale, void* out, int64_t o_tok_stride,
+                                int64_t o_head_stride, void* workspace, size_t workspace_bytes,
+                                coopt_stream_t stream);
+/* Rows per KV head of the query windows such a call runs in: 128, 64, or 0 where its items
+ * are not cut into windows. */
+int coopt_verify_attention_window_rows(int kv_dtype, int B, int Hq, int Hkv, int max_seqlen_q,
+                                       int max_seqlen_k, int64_t total_q);
 
 /*
  * The qkv epilogue and the verification attention of one layer in one launch: replaces

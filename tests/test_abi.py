@@ -106,6 +106,35 @@ def test_verify_attention_reports_small_workspace(lib):
     assert rc == _lib.COOPT_EWORKSPACE and "workspace" in _lib.last_error()
 
 
+# Windowed attention calls and the us they take in query windows of 64 and of 128 rows (MI355X, head
+# dim 128, the longest context max_k): INT8?, B, Hq, Hkv, max_q, max_k, query rows.
+WINDOWED = [
+    (0, 1, 32, 8, 512, 512, 512, 14.8, 21.1), (0, 1, 32, 8, 512, 4096, 512, 65.1, 119.5),
+    (0, 1, 32, 8, 512, 16384, 512, 240.6, 438.4), (1, 1, 32, 8, 512, 16384, 512, 321.4, 530.6),
+    (0, 1, 32, 8, 2048, 4096, 2048, 197.4, 142.7), (1, 1, 32, 8, 2048, 16384, 2048, 1163.8, 740.5),
+    (0, 5, 32, 8, 256, 4096, 276, 68.7, 120.6), (0, 17, 32, 8, 33, 4096, 113, 67.4, 121.5),
+    (0, 17, 32, 8, 64, 4096, 144, 182.0, 123.8), (0, 17, 32, 8, 512, 16384, 592, 712.9, 448.8),
+    (0, 32, 32, 8, 33, 4096, 188, 130.7, 166.8), (0, 32, 32, 8, 512, 1000, 667, 105.7, 31.8),
+    (0, 4, 32, 8, 17, 4096, 68, 64.3, 119.9), (0, 4, 32, 8, 512, 4096, 2048, 240.2, 166.2),
+    (0, 16, 32, 8, 128, 4096, 2048, 255.1, 177.6), (0, 40, 32, 8, 256, 256, 10240, 172.9, 75.7),
+    (1, 40, 32, 8, 128, 4096, 5120, 862.0, 506.0),
+    (0, 33, 32, 4, 1553, 1553, 1681, 114.1, 58.2), (0, 6, 32, 4, 107, 3996, 244, 63.5, 118.6),
+]
+
+
+def test_window_rows_are_the_faster_ones(lib):
+    for int8, B, Hq, Hkv, max_q, max_k, rows, t64, t128 in WINDOWED:
+        got = lib.coopt_verify_attention_window_rows(_lib.DT_I8 if int8 else _lib.DT_BF16, B, Hq, Hkv,
+                                                     max_q, max_k, rows)
+        assert got == (128 if t128 < t64 else 64), (int8, B, Hq, Hkv, max_q, max_k, rows)
+    # not windowed; refused shapes; rows unknown or short count as one a sequence
+    q = lib.coopt_verify_attention_window_rows
+    assert q(_lib.DT_BF16, 4, 32, 8, 16, 4096, 64) == 0 and q(_lib.DT_BF16, 4, 32, 8, 17, 4096, 68) == 64
+    assert q(_lib.DT_BF16, 4, 130, 2, 17, 4096, 68) == 0 and q(_lib.DT_BF16, 0, 32, 8, 17, 4096, 0) == 0
+    for B, max_q in ((1, 512), (16, 128), (70, 20)):
+        assert q(_lib.DT_BF16, B, 32, 8, max_q, 4096, 0) == q(_lib.DT_BF16, B, 32, 8, max_q, 4096, max_q + B - 1)
+
+
 def test_accept_sample_rejects_bad_arguments(lib):
     assert "logits_dtype" in _err(lib.coopt_accept_sample(5, 16, 100, 0, 0, 16, 100, 0, 16, 0,
                                                           16, 16, 1.0, 2, 4, 100, 16, 16, 0, 16,

@@ -469,6 +469,21 @@ def test_rows_past_the_end_and_many_splits(dev, kv, D, ctx, q_lens):
     assert excess <= (TOL_BF16 if kv == "auto" else TOL_INT8)
 
 
+@pytest.fixture
+def long_windows(monkeypatch):
+    """Calls that run in query windows take the 128-row ones (prefill_attn_kernel), as with far more
+    query rows; the returned check says whether a batch's call does."""
+    lib, rows = M._lib.load(), 1 << 24
+    call = lib.coopt_verify_attention_rows
+    monkeypatch.setattr(lib, "coopt_verify_attention_rows", lambda *a: call(*a[:26], rows, *a[27:]))
+
+    def check(kv, Hq, Hkv, ctx, q_lens):
+        code = M._lib.DT_I8 if kv == "int8" else M._lib.DT_BF16
+        max_k = max(c + n for c, n in zip(ctx, q_lens))
+        assert lib.coopt_verify_attention_window_rows(code, len(ctx), Hq, Hkv, max(q_lens), max_k, rows) == 128
+    return check
+
+
 @pytest.mark.parametrize("kv,D,G,ctx,q_lens,bs", [
     ("auto", 128, 4, [0, 37, 900, 5], [513, 1, 5, 64], 16),       # 17 windows, the last of 1 row
     ("int8", 128, 4, [0, 37, 900, 5], [513, 1, 5, 65], 16),
@@ -477,9 +492,10 @@ def test_rows_past_the_end_and_many_splits(dev, kv, D, ctx, q_lens):
     ("int8", 128, 4, [10] * 3 + [300] * 67, [64, 1, 33] + [2] * 67, 16),  # 70 sequences: grid order
     ("auto", 64, 4, list(range(0, 320, 10)), [64] * 32, 16),      # 32 sequences of 256 rows
 ])
-def test_long_chunks_match_the_oracle(dev, kv, D, G, ctx, q_lens, bs):
-    """The prefill kernel (2048 rows per KV head, or 256 with 32 sequences): window and stage
-    remainders, mixed batches, stale rows past the end.  Tolerances as at the top."""
+def test_long_chunks_match_the_oracle(dev, long_windows, kv, D, G, ctx, q_lens, bs):
+    """The prefill kernel: window and stage remainders, mixed batches, stale rows past the end.
+    Tolerances as at the top."""
+    long_windows(kv, 4 * G, 4, ctx, q_lens)
     pool = Pool(ctx, q_lens, 4 * G, 4, D, dev, kv=kv, bs=bs, seed=D + G, slack=2)
     for t in (pool.kc, pool.vc) if kv == "auto" else (pool.ks, pool.vs):
         b = len(ctx) - 1                                          # rows past one sequence's end
