@@ -71,7 +71,7 @@ SIGNATURES = {
     "coopt_verify_attention_rows": (_i, [_i, _p, _i64, _i64, _p, _p, _i64, _i64, _i64, _p, _p,
                                          _i64, _i64, _i64, _p, _i64, _p, _p, _i, _i, _i, _i, _i,
                                          _i64, _i, _i, _i64, _f, _p, _i64, _i64, _p, _sz, _p]),
-    "coopt_verify_attention_window_rows": (_i, [_i, _i, _i, _i, _i, _i, _i64]),
+    "coopt_verify_attention_window_rows": (_i, [_i, _i, _i, _i, _i, _i, _i, _i64]),
     "coopt_accept_sample_workspace": (_sz, [_i, _i, _i]),
     "coopt_accept_sample": (_i, [_i, _p, _i64, _p, _i, _p, _i64, _p, _p, _p, _p, _p, _f, _i, _i,
                                  _i, _p, _p, _p, _p, _sz, _p]),

@@ -105,6 +105,7 @@ struct AttnArgs {
   // + w) * Hkv + hkv, one split per window (prefill_attn_kernel orders them itself).
   int qwin, nwin;
   int prefill;  // host side: prefill_attn_kernel takes the windows
+  int alone;    // host side: one block a CU (alone_lds)
   // Fused qkv epilogue (coopt_verify_attention_qkv): qkv_mode 0 = q is given; 1 = bf16 qkv
   // projection rows; 2 = their fp32 split-K partials.  The block computes its own q rows
   // (RoPE'd, straight into LDS) and writes its KV head's new K/V to the cache first.
@@ -1597,6 +1598,7 @@ struct AttnShape {
   int rmax;        // rows per (item, KV head): G * max_seqlen_q, or G * qwin when windowed
   int qwin, nwin;  // windowed: rows per window and windows per sequence (else 0, 0)
   bool prefill;    // windowed, by prefill_attn_kernel
+  bool alone;      // windowed, a block on each CU holds them all (alone_lds)
 };
 
 constexpr int kMaxRows = 64;
@@ -1607,16 +1609,19 @@ constexpr int kMaxRows = 64;
 //                        block of the grid without rows.  Blocks go to the 32 pairs of XCD and
 //                        shader engine in turn, so where the sequences' first windows lie a
 //                        multiple apart in the grid, the items of one window share a part of the pairs
-//                        (a chunk of 64 tokens with 16 items of 5, 4096 keys: 182 us, of 33 tokens: 67)
+//                        (a chunk of 64 tokens with 16 items of 5, 4096 keys: 182 us, of 33 tokens: 67).
+//                        Beyond one round 0.8 of that at head dim 64
 //   prefill_attn_kernel  6.5 + 0.038 k per round of 512 windows (two on a CU), by halves; 1.4 ns per
 //                        block without rows; it packs its windows unless B > kPlanSeqs
 // Fitted to 2784 batches of 1 to 70 sequences, chunks of 17 to 2100 tokens, 17 to 18000 keys, 1 to 16 KV
-// heads, G 1 to 8, bf16 and INT8, head dims 64 and 128: against verify_attn_kernel for all of them the
-// times' mean is 0.77 (the faster kernel each time: 0.76), 16 batches are more than 3 % slower, the
-// worst 1.18 (prefill_attn_kernel for all: 1.97).  us, verify / prefill, bf16, 32/8 heads of 128: a chunk of 512
+// heads, G 1 to 8, bf16 and INT8, head dims 64 and 128. On 1000 further ones the call takes 0.79 of the
+// time of verify_attn_kernel for all (one block a CU) in the mean; 5 are more than 3 % slower, the
+// worst 1.22 (one chunk over its own keys). us, verify / prefill, bf16, 32/8 heads of 128: a chunk of 512
 // tokens over 512 keys 14.8 / 21.1, over 16384 240 / 438, with 16 items of 5 over 16384 713 / 449; 1024
 // over 4096 114 / 120; 2048 over 4096 197 / 143; 16 chunks of 256 over 4096 504 / 347.
-bool prefill_is_faster(int B, int G, int Hkv, int max_seqlen_q, int max_seqlen_k, int64_t total_q, bool int8) {
+// `one_round`: verify_attn_kernel's windows are estimated to run in one round (alone_lds).
+bool prefill_is_faster(int B, int G, int Hkv, int D, int max_seqlen_q, int max_seqlen_k, int64_t total_q,
+                       bool int8, bool& one_round) {
   constexpr double kCus = 256;
   const int64_t others = total_q > max_seqlen_q ? total_q - max_seqlen_q : 0;  // rows of the other sequences
   struct Grid {
@@ -1648,19 +1653,21 @@ bool prefill_is_faster(int B, int G, int Hkv, int max_seqlen_q, int max_seqlen_k
   double p_rounds = fmax(1.0, 0.5 * ceil((p.longest * seen + p.rest) / kCus));
   if (B > 1) v_rounds = fmax(v_rounds, ceil(0.4 * v.longest / kCus + v.firsts / (kCus * v.pairs)));
   if (B > kPlanSeqs) p_rounds = fmax(p_rounds, ceil(0.5 * p.firsts / (kCus * p.pairs)));
-  const double v_us = v_rounds * (8.0 + (int8 ? 0.0185 : 0.0135) * k) + 0.005 * v.empty;
+  one_round = v_rounds <= 1.0;
+  const double more = D == 64 && !one_round ? 0.8 : 1.0;
+  const double v_us = more * v_rounds * (8.0 + (int8 ? 0.0185 : 0.0135) * k) + 0.005 * v.empty;
   const double p_us = p_rounds * (6.5 + 0.038 * k) + 0.0014 * p.empty;
   return 1.03 * p_us < v_us;
 }
 
 // total_q: the call's query rows, 0 if unknown (one row for every sequence but the longest then);
 // it and int8 decide between the window kernels only, not any workspace.
-AttnShape attn_shape(int B, int G, int Hkv, int max_seqlen_q, int max_seqlen_k, int64_t total_q, bool int8) {
+AttnShape attn_shape(int B, int G, int Hkv, int D, int max_seqlen_q, int max_seqlen_k, int64_t total_q, bool int8) {
   AttnShape s{};
   if (G * static_cast<int64_t>(max_seqlen_q) > kMaxRows) {
     // longer items run in query windows of kMaxRows (verify_attn_kernel: a wave's tiles are its
     // own, which suits few windows) or kPrefillRows rows (prefill_attn_kernel)
-    s.prefill = prefill_is_faster(B, G, Hkv, max_seqlen_q, max_seqlen_k, total_q, int8);
+    s.prefill = prefill_is_faster(B, G, Hkv, D, max_seqlen_q, max_seqlen_k, total_q, int8, s.alone);
     s.qwin = (s.prefill ? kPrefillRows : kMaxRows) / G;
     s.nwin = (max_seqlen_q + s.qwin - 1) / s.qwin;
     s.rmax = G * s.qwin;
@@ -1699,6 +1706,16 @@ constexpr bool fused_ok(int D, bool int8, int RT) {
   return RT >= 1 && RT <= kFusedMaxRT && (int8 || D != 128 || RT == 1);
 }
 
+// LDS asked for beside a 64-row block's own (76 KB at head dim 64, bf16), so that no second one fits its
+// CU.  Two a CU raise the rate (batches of more than 256 windows: 0.73 of the time), but windows that a
+// block on each CU would hold then double up on some of them: 5 sequences with one chunk of 286 tokens
+// over 1500 keys, 176 windows among 720 blocks, 25.4 us with two a CU and 21.7 with one.  360 batches,
+// this rule against one a CU for all: 0.84 in the mean, 1.06 at worst (two for all: 1.27).
+template <int D, bool INT8>
+unsigned alone_lds(const AttnArgs& a) {
+  return D == 64 && !INT8 && a.alone ? 8192u : 0u;
+}
+
 template <int D, bool INT8, bool SC>
 int launch_rt(int RT, const AttnArgs& a, dim3 grid, hipStream_t s) {
   if (a.qkv_mode) {
@@ -1720,7 +1737,7 @@ int launch_rt(int RT, const AttnArgs& a, dim3 grid, hipStream_t s) {
     case 1: hipLaunchKernelGGL((verify_attn_kernel<D, INT8, 1, SC, 0>), grid, dim3(64 * waves_for(1)), 0, s, ATTN_LEAD(a), a); break;
     case 2: hipLaunchKernelGGL((verify_attn_kernel<D, INT8, 2, SC, 0>), grid, dim3(64 * waves_for(2)), 0, s, ATTN_LEAD(a), a); break;
     case 3: hipLaunchKernelGGL((verify_attn_kernel<D, INT8, 3, SC, 0>), grid, dim3(64 * waves_for(3)), 0, s, ATTN_LEAD(a), a); break;
-    case 4: hipLaunchKernelGGL((verify_attn_kernel<D, INT8, 4, SC, 0>), grid, dim3(64 * waves_for(4)), 0, s, ATTN_LEAD(a), a); break;
+    case 4: hipLaunchKernelGGL((verify_attn_kernel<D, INT8, 4, SC, 0>), grid, dim3(64 * waves_for(4)), (alone_lds<D, INT8>(a)), s, ATTN_LEAD(a), a); break;
     default: return COOPT_EINVAL;
   }
   int rc = coopt::check_launch("coopt_verify_attention");
@@ -1748,7 +1765,7 @@ extern "C" size_t coopt_verify_attention_workspace(int B, int Hq, int Hkv, int D
   if (B <= 0 || Hkv <= 0 || Hq <= 0 || Hq % Hkv || Hq / Hkv > kMaxRows || max_seqlen_q <= 0 ||
       max_seqlen_k <= 0)
     return 0;
-  const AttnShape sh = attn_shape(B, Hq / Hkv, Hkv, max_seqlen_q, max_seqlen_k, 0, false);
+  const AttnShape sh = attn_shape(B, Hq / Hkv, Hkv, D, max_seqlen_q, max_seqlen_k, 0, false);
   if (sh.nwin > 0) return 256;  // one split per window: no partials
   return attn_ws_layout(B, Hkv, D, sh.rmax, sh.max_splits).total;
 }
@@ -1857,7 +1874,7 @@ int verify_attention_impl(const char* who, const FusedQkv* fz, int kv_dtype, con
   a.out = static_cast<uint16_t*>(out);
   a.o_ts = o_tok_stride;
   a.o_hs = o_head_stride;
-  const AttnShape shape = attn_shape(B, G, Hkv, max_seqlen_q, max_seqlen_k, total_q, int8);
+  const AttnShape shape = attn_shape(B, G, Hkv, D, max_seqlen_q, max_seqlen_k, total_q, int8);
   // grid limits: 2^32 work-items along x, 65535 blocks along z
   ATTN_REQUIRE(shape.nwin == 0 || static_cast<int64_t>(B) * shape.nwin * Hkv < (int64_t{1} << 24),
                "too many query windows for one launch");
@@ -1866,6 +1883,7 @@ int verify_attention_impl(const char* who, const FusedQkv* fz, int kv_dtype, con
   a.qwin = shape.qwin;
   a.nwin = shape.nwin;
   a.prefill = shape.prefill;
+  a.alone = shape.alone;
   a.split = shape.split;
   a.max_splits = shape.max_splits;
   a.B = B;
@@ -1970,12 +1988,12 @@ extern "C" int coopt_verify_attention_rows(int kv_dtype, const void* q, int64_t 
                                workspace_bytes, stream);
 }
 
-extern "C" int coopt_verify_attention_window_rows(int kv_dtype, int B, int Hq, int Hkv, int max_seqlen_q,
-                                                 int max_seqlen_k, int64_t total_q) {
+extern "C" int coopt_verify_attention_window_rows(int kv_dtype, int B, int Hq, int Hkv, int D,
+                                                 int max_seqlen_q, int max_seqlen_k, int64_t total_q) {
   if (B <= 0 || Hkv <= 0 || Hq <= 0 || Hq % Hkv || Hq / Hkv > kMaxRows || max_seqlen_q <= 0 ||
       max_seqlen_k <= 0)
     return 0;
-  const AttnShape s = attn_shape(B, Hq / Hkv, Hkv, max_seqlen_q, max_seqlen_k, total_q, kv_dtype == COOPT_DT_I8);
+  const AttnShape s = attn_shape(B, Hq / Hkv, Hkv, D, max_seqlen_q, max_seqlen_k, total_q, kv_dtype == COOPT_DT_I8);
   return s.nwin == 0 ? 0 : s.prefill ? kPrefillRows : kMaxRows;
 }
 
@@ -1987,7 +2005,7 @@ extern "C" int coopt_verify_attention_qkv_supported(int kv_dtype, int B, int Hq,
   const int G = Hq / Hkv;
   if (static_cast<int64_t>(G) * max_seqlen_q > kMaxRows) return 0;
   if (!fused_ok(D, kv_dtype == COOPT_DT_I8, (G * max_seqlen_q + 15) / 16)) return 0;
-  return attn_shape(B, G, Hkv, max_seqlen_q, max_seqlen_k, 0, false).max_splits == 1 ? 1 : 0;
+  return attn_shape(B, G, Hkv, D, max_seqlen_q, max_seqlen_k, 0, false).max_splits == 1 ? 1 : 0;
 }
 
 extern "C" int coopt_verify_attention_qkv(

@@ -287,8 +287,8 @@ int coopt_verify_attention_rows(int kv_dtype,
                                 coopt_stream_t stream);
 /* Rows per KV head of the query windows such a call runs in: 128, 64, or 0 where its items
  * are not cut into windows. */
-int coopt_verify_attention_window_rows(int kv_dtype, int B, int Hq, int Hkv, int max_seqlen_q,
-                                       int max_seqlen_k, int64_t total_q);
+int coopt_verify_attention_window_rows(int kv_dtype, int B, int Hq, int Hkv, int D,
+                                       int max_seqlen_q, int max_seqlen_k, int64_t total_q);
 
 /*
  * The qkv epilogue and the verification attention of one layer in one launch: replaces

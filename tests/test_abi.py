@@ -124,15 +124,15 @@ WINDOWED = [
 
 def test_window_rows_are_the_faster_ones(lib):
     for int8, B, Hq, Hkv, max_q, max_k, rows, t64, t128 in WINDOWED:
-        got = lib.coopt_verify_attention_window_rows(_lib.DT_I8 if int8 else _lib.DT_BF16, B, Hq, Hkv,
+        got = lib.coopt_verify_attention_window_rows(_lib.DT_I8 if int8 else _lib.DT_BF16, B, Hq, Hkv, 128,
                                                      max_q, max_k, rows)
         assert got == (128 if t128 < t64 else 64), (int8, B, Hq, Hkv, max_q, max_k, rows)
     # not windowed; refused shapes; rows unknown or short count as one a sequence
     q = lib.coopt_verify_attention_window_rows
-    assert q(_lib.DT_BF16, 4, 32, 8, 16, 4096, 64) == 0 and q(_lib.DT_BF16, 4, 32, 8, 17, 4096, 68) == 64
-    assert q(_lib.DT_BF16, 4, 130, 2, 17, 4096, 68) == 0 and q(_lib.DT_BF16, 0, 32, 8, 17, 4096, 0) == 0
+    assert q(_lib.DT_BF16, 4, 32, 8, 128, 16, 4096, 64) == 0 and q(_lib.DT_BF16, 4, 32, 8, 128, 17, 4096, 68) == 64
+    assert q(_lib.DT_BF16, 4, 130, 2, 128, 17, 4096, 68) == 0 and q(_lib.DT_BF16, 0, 32, 8, 128, 17, 4096, 0) == 0
     for B, max_q in ((1, 512), (16, 128), (70, 20)):
-        assert q(_lib.DT_BF16, B, 32, 8, max_q, 4096, 0) == q(_lib.DT_BF16, B, 32, 8, max_q, 4096, max_q + B - 1)
+        assert q(_lib.DT_BF16, B, 32, 8, 64, max_q, 4096, 0) == q(_lib.DT_BF16, B, 32, 8, 64, max_q, 4096, max_q + B - 1)
 
 
 def test_accept_sample_rejects_bad_arguments(lib):

@@ -477,10 +477,10 @@ def long_windows(monkeypatch):
     call = lib.coopt_verify_attention_rows
     monkeypatch.setattr(lib, "coopt_verify_attention_rows", lambda *a: call(*a[:26], rows, *a[27:]))
 
-    def check(kv, Hq, Hkv, ctx, q_lens):
+    def check(kv, Hq, Hkv, D, ctx, q_lens):
         code = M._lib.DT_I8 if kv == "int8" else M._lib.DT_BF16
         max_k = max(c + n for c, n in zip(ctx, q_lens))
-        assert lib.coopt_verify_attention_window_rows(code, len(ctx), Hq, Hkv, max(q_lens), max_k, rows) == 128
+        assert lib.coopt_verify_attention_window_rows(code, len(ctx), Hq, Hkv, D, max(q_lens), max_k, rows) == 128
     return check
 
 
@@ -495,7 +495,7 @@ def long_windows(monkeypatch):
 def test_long_chunks_match_the_oracle(dev, long_windows, kv, D, G, ctx, q_lens, bs):
     """The prefill kernel: window and stage remainders, mixed batches, stale rows past the end.
     Tolerances as at the top."""
-    long_windows(kv, 4 * G, 4, ctx, q_lens)
+    long_windows(kv, 4 * G, 4, D, ctx, q_lens)
     pool = Pool(ctx, q_lens, 4 * G, 4, D, dev, kv=kv, bs=bs, seed=D + G, slack=2)
     for t in (pool.kc, pool.vc) if kv == "auto" else (pool.ks, pool.vs):
         b = len(ctx) - 1                                          # rows past one sequence's end
