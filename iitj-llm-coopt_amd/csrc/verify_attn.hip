@@ -72,6 +72,9 @@ constexpr int kThreads = 256;  // merge kernel
 // Waves per attention block: 8 (one block per CU at two waves per SIMD, i.e. at most 256
 // registers per lane) while the accumulators and two tile buffers fit that (RT <= 3), else 4.
 constexpr int waves_for(int RT) { return RT <= 3 ? 8 : 4; }
+// Blocks that share a CU: two with 4 waves at head dim 64 and bf16 (76 KB of LDS, at most 256 registers
+// asked for), where batches of many query windows take 0.63 to 0.8 of the time; see alone_lds.
+constexpr int blocks_per_cu(int D, bool int8, int RT) { return D == 64 && !int8 && RT == 4 ? 2 : 1; }
 constexpr int kTileKeys = 32;
 constexpr float kLog2e = 1.4426950408889634f;
 
@@ -263,7 +266,7 @@ __device__ void plan_item(const AttnArgs& a, int lane, int* out) {
 // (a run-time choice of input made the compiler wait for every earlier load where the two
 // input paths joined).
 template <int D, bool INT8, int RT, bool SC, int FUSED>
-__global__ __launch_bounds__(64 * waves_for(RT), 1) void verify_attn_kernel(
+__global__ __launch_bounds__(64 * waves_for(RT), blocks_per_cu(D, INT8, RT)) void verify_attn_kernel(
     const int32_t* cu_p, const int32_t* sl_p, const int32_t* bt_p, int64_t bt_stride, int split,
     int bs_shift, int mode, AttnArgs a) {
   using Raw = RawTile<D, INT8>;
@@ -309,9 +312,8 @@ __global__ __launch_bounds__(64 * waves_for(RT), 1) void verify_attn_kernel(
   typedef const __attribute__((address_space(4))) int32_t* const_i32_ptr;
   const int64_t bt_last = bt_stride - 1;
   // The pages of the wave's first tile of piece sidx of sequence b, looked up before L is
-  // known, so not clamped to the last key's page: a half tile past the end may get whatever
-  // page its table entry names, clamped into the pool, and clear_tail drops what is read there
-  // (the index is kept inside the table row regardless).
+  // known: they are used only if that tile is full, i.e. all its keys are < L, where no
+  // clamp to L - 1 applies (the index is kept inside the table row regardless).
   auto first_pages = [&](int b, int sidx, int32_t& p0, int32_t& p1) {
     const const_i32_ptr tb = (const_i32_ptr)(bt_p + static_cast<int64_t>(b) * bt_stride);
     const int kb = sidx * split + wave * kTileKeys;
@@ -490,7 +492,9 @@ __global__ __launch_bounds__(64 * waves_for(RT), 1) void verify_attn_kernel(
   };
 
   // Issue every load of tile `t` (pages pg0/pg1).  Page bases are wave-uniform (scalar);
-  // lanes add 32-bit byte offsets, fixed for the whole loop.
+  // lanes add 32-bit byte offsets.  Full tiles (every key < L) use offsets fixed for the
+  // whole loop; the last, partial tile clamps each key to L - 1, so no row past the
+  // sequence is read.
   const int c_ts = static_cast<int>(a.c_ts), s_ts = static_cast<int>(a.s_ts);
   const uint32_t k_lane = kElt * l16 * c_ts + 16 * grp;
   uint32_t v_lane[4];
@@ -513,9 +517,10 @@ __global__ __launch_bounds__(64 * waves_for(RT), 1) void verify_attn_kernel(
       load_words<Raw::kVWords>(vp + off, raw.v[kt * 4 + i]);
     }
   };
+  // a full tile: every key < L
   // INT8: the scales are issued first, so the V-scale check of a loaded tile (vcheck) waits
   // only for them and leaves the tile's K/V loads in flight.
-  auto load_tile = [&](Raw& raw, int t, int64_t pg0, int64_t pg1) {
+  auto load_full = [&](Raw& raw, int t, int64_t pg0, int64_t pg1) {
     const int kb = k_begin + t * kTileKeys;
     if constexpr (INT8) {
 #pragma unroll
@@ -546,21 +551,32 @@ __global__ __launch_bounds__(64 * waves_for(RT), 1) void verify_attn_kernel(
       issue(raw, kt, kbase + kElt * r, vbase + kElt * r, k_lane, v_lane);
     }
   };
-  // The split's last tile when the sequence ends inside it: loaded like the others (the rows
-  // past the end lie in the same page, or in some page of the pool), then the values of the
-  // keys past the end are zeroed -- their probabilities are 0, but 0 times whatever a row that
-  // was never written holds need not be -- and with them the V scales vcheck looks at.
-  auto clear_tail = [&](Raw& raw, int t) {
-    // keys of the tile inside the split, from the lane's first one on (the asm keeps eight
-    // comparands from being held in registers through the loop)
-    int left = k_end - (k_begin + t * kTileKeys) - grp * 4;
-    asm volatile("" : "+v"(left));
+  // the split's last tile when it ends inside a tile: keys clamped to L - 1
+  auto load_partial = [&](Raw& raw, int t, int64_t pg0, int64_t pg1) {
+    const int kb = k_begin + t * kTileKeys;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const uint32_t keep = (j >> 2) * 16 + (j & 3) < left ? 0xffffffffu : 0u;
+    for (int kt = 0; kt < 2; ++kt) {
+      const int64_t pg = kt ? pg1 : pg0;
+      const int sub = kb + kt * 16;
+      const int64_t row0 = pg * a.c_bs + head_off;
+      const int ktk = min(sub + l16, L - 1) & bs_mask;
+      const uint32_t ko = kElt * ktk * c_ts + 16 * grp;
+      uint32_t vo[4], tk[4];
 #pragma unroll
-      for (int w = 0; w < Raw::kVWords; ++w) raw.v[j][w] &= keep;
-      if constexpr (INT8) raw.vs[j >> 2][(j >> 1) & 1] &= (j & 1) ? (keep | 0xffffu) : (keep | 0xffff0000u);
+      for (int i = 0; i < 4; ++i) {
+        tk[i] = min(sub + grp * 4 + i, L - 1) & bs_mask;
+        vo[i] = kElt * (tk[i] * c_ts + l16 * kDt);
+      }
+      issue(raw, kt, kbase + kElt * row0, vbase + kElt * row0, ko, vo);
+      if constexpr (INT8) {
+        const uint16_t* ksp = a.ks + pg * a.s_bs + shead_off;
+        const uint16_t* vsp = a.vs + pg * a.s_bs + shead_off;
+        raw.ks[kt] = ksp[ktk * s_ts];
+        uint32_t vh[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) vh[i] = vsp[tk[i] * s_ts];
+        raw.vs[kt] = u32x2_t{vh[0] | (vh[1] << 16), vh[2] | (vh[3] << 16)};
+      }
     }
   };
 
@@ -771,73 +787,83 @@ __global__ __launch_bounds__(64 * waves_for(RT), 1) void verify_attn_kernel(
   };
 
   // ---- the wave's tiles: double-buffered (the next tile's loads in flight while the current
-  // one is computed) or, for large row counts, one at a time ----
+  // one is computed) or, for large row counts, one at a time; then the partial tile ----
   // Wave w takes tiles w, w + kWaves, w + 2 kWaves, ... (a fixed assignment keeps the result
-  // bit-reproducible: each wave's sum covers the same keys on every call).  The split's partial
-  // last tile is one of them: its loads are the last ones issued in the wave's loop, and it is
-  // computed behind the loop (loaded there as well, it cost its wave a memory round trip: 1
-  // sequence, 717 keys, unsplit: 11.6 us, 11.3 like this).
+  // bit-reproducible: each wave's sum covers the same keys on every call); the wave whose
+  // sequence reaches nfull also takes the split's partial tile.
   const int nfull = (k_end - k_begin) / kTileKeys;
-  const bool own_partial = nfull < ntiles && nfull % kWaves == wave;
-  const int tlast = own_partial ? nfull : nfull - 1;  // the last tile the wave may load
   auto pages = [&](int t, int64_t& p0, int64_t& p1) {
     const int kb = k_begin + t * kTileKeys;
     p0 = page_of(kb);
     p1 = page_of(kb + 16);
   };
-  Raw bufA;
+  bool own_partial = wave == nfull;
+  int next_t = wave + kWaves;
+  auto grab = [&]() {
+    const int v = next_t;
+    next_t += kWaves;
+    own_partial |= v == nfull;
+    return v;
+  };
   if constexpr (DB) {
-    // Loads inside the loop are unconditional (an index past the last tile repeats it,
+    // Loads inside the loop are unconditional (an index past the last full tile repeats it,
     // already cached, and is never computed), so each compute waits only for its own
     // buffer's loads and the other buffer's stay in flight.
-    Raw bufB;
+    Raw bufA, bufB;
+    const int tlast = nfull - 1;
     int tA = wave;
     int64_t nx0 = 0, nx1 = 0;  // pages of the wave's next tile to load
     // fused: a first tile holding keys this launch writes ([L - n, L)) loads after the barrier
     const bool defer = fused && k_begin + (tA + 1) * kTileKeys > L - n;
-    if (tA <= tlast && !defer) load_tile(bufA, tA, first_pg0, first_pg1);
+    if (tA < nfull && !defer) load_full(bufA, tA, first_pg0, first_pg1);
     stage_q();  // the Q loads complete while the first tile's are in flight
-    if (tA <= tlast && defer) load_tile(bufA, tA, first_pg0, first_pg1);
+    if (tA < nfull && defer) load_full(bufA, tA, first_pg0, first_pg1);
     if (tA < nfull) {
       vcheck(bufA);
-      int tB = tA + kWaves;
+      int tB = grab();
       pages(min(tB, tlast), nx0, nx1);
       for (;;) {
-        load_tile(bufB, min(tB, tlast), nx0, nx1);
-        const int tA2 = tB + kWaves;
+        load_full(bufB, min(tB, tlast), nx0, nx1);
+        const int tA2 = tB < nfull ? grab() : nfull;
         pages(min(tA2, tlast), nx0, nx1);
         compute_tile(bufA, tA);
-        if (tB >= nfull) {
-          bufA = bufB;
-          break;
-        }
         vcheck(bufB);
-        load_tile(bufA, min(tA2, tlast), nx0, nx1);
-        const int tB2 = tA2 + kWaves;
+        if (tB >= nfull) break;
+        load_full(bufA, min(tA2, tlast), nx0, nx1);
+        const int tB2 = tA2 < nfull ? grab() : nfull;
         pages(min(tB2, tlast), nx0, nx1);
         compute_tile(bufB, tB);
-        if (tA2 >= nfull) break;
         vcheck(bufA);
+        if (tA2 >= nfull) break;
         tA = tA2;
         tB = tB2;
       }
     }
   } else {
-    int64_t nx0 = first_pg0, nx1 = first_pg1;
-    stage_q();
+    Raw buf;
+    int64_t nx0 = 0, nx1 = 0;
     int t = wave;
-    for (; t < nfull; t += kWaves) {
-      load_tile(bufA, t, nx0, nx1);
-      if (t + kWaves <= tlast) pages(t + kWaves, nx0, nx1);
-      vcheck(bufA);
-      compute_tile(bufA, t);
+    if (t < nfull) {
+      nx0 = first_pg0;
+      nx1 = first_pg1;
     }
-    if (own_partial) load_tile(bufA, t, nx0, nx1);
+    stage_q();
+    while (t < nfull) {
+      load_full(buf, t, nx0, nx1);
+      const int tn = grab();
+      if (tn < nfull) pages(tn, nx0, nx1);
+      vcheck(buf);
+      compute_tile(buf, t);
+      t = tn;
+    }
   }
-  if (own_partial) {
-    clear_tail(bufA, nfull);
-    vcheck(bufA);
-    compute_tile(bufA, nfull);
+  if (nfull < ntiles && own_partial) {
+    Raw buf;
+    int64_t p0, p1;
+    pages(nfull, p0, p1);
+    load_partial(buf, nfull, p0, p1);
+    vcheck(buf);
+    compute_tile(buf, nfull);
   }
   // ---- merge the waves ----
   // the wave's o and l are relative to 2^(m_run + e_v) (e_v = 0 for bf16 KV)
