@@ -46,14 +46,14 @@ def test_no_kernel_spills_to_scratch(tmp_path):
 
 
 @pytest.mark.skipif(HIPCC is None, reason="hipcc not installed")
-def test_projection_barriers_are_reached_by_every_wave(tmp_path):
-    """The projection kernels' waves branch on their index before the last barrier (the fused
-    SiLU's exchange): no execution mask is narrowed up to there, so no barrier lies in an arm
-    that a wave might skip or pass through with its lanes off."""
+def test_fused_silu_barriers_are_reached_by_every_wave(tmp_path):
+    """The fused gate_up + SiLU kernels' waves branch on their index before the last barrier (the
+    exchange of row tiles): no execution mask is narrowed up to there, so no barrier lies in an
+    arm that a wave might skip or pass through with its lanes off."""
     resources("linear.hip", str(tmp_path))
     kernels, name = {}, None
     for line in open(os.path.join(str(tmp_path), "linear.hip.s")):
-        m = re.match(r"(_Z\w*linear_kernel\w*):", line)
+        m = re.match(r"(_Z\w*linear_kernelI(?:Li\d+E){4}Lb1ELb[01]ELb1E\w*):", line)  # SILU, the last
         if m:
             name = m.group(1)
             kernels[name] = []
@@ -61,7 +61,7 @@ def test_projection_barriers_are_reached_by_every_wave(tmp_path):
             name = None
         elif name:
             kernels[name].append(line.split(";")[0])
-    assert len(kernels) > 20, list(kernels)
+    assert len(kernels) == 8, list(kernels)
     narrowed = re.compile(r"_saveexec_b64|s_\w+_b64 exec,|v_cmpx_")
     bad = {}
     for k, lines in kernels.items():
