@@ -148,12 +148,14 @@ __global__ __launch_bounds__(64 * WAVES) void linear_kernel(
 #pragma unroll
       for (int j = 0; j < 4; ++j) wr[nt][j] = ldg16<NT>(wrow[nt] + s * kWStep + kWChunk * j);
   };
-  // Row-major weights: behind a branch, taken or not, 4096 x 4096 of up to 48 rows take 8.25 us instead of
-  // 8.55, 2048 x 2048 of 48 and 64 rows 5.9 instead of 6.1; packed ones are up to 5 % faster without it.
+  // Behind a branch, taken or not, where W is row-major or a slice is short and the rows few: 4096 x 4096
+  // of up to 48 rows, row-major, 8.25 us instead of 8.55, packed (8 steps a slice) 7.9 instead of
+  // 8.1.  The other packed ones are up to 5 % faster without it.
+  constexpr bool kPlainStore = PK && (NT || MT > 4 || SILU);
   auto store_x = [&](int buf, const u32x4_t (&xr)[kRounds]) {
 #pragma unroll
     for (int r = 0; r < kRounds; ++r)
-      if (PK || r * kRowsPerRound + xr_row < MT * 16)
+      if (kPlainStore || r * kRowsPerRound + xr_row < MT * 16)
         *reinterpret_cast<u32x4_t*>(&xs[buf][(r * kRowsPerRound + xr_row) * kPitch + xr_col * 2]) = xr[r];
   };
 
