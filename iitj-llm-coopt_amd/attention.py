@@ -18,6 +18,7 @@ the GPU, of 128/(Hq/Hkv) rows in a kernel that stages K and V in LDS for the win
 """
 import functools
 import math
+import operator
 
 import torch
 
@@ -30,10 +31,16 @@ _WS = _lib.WorkspaceCache()
 
 
 @functools.lru_cache(maxsize=1024)   # a pure function of the sizes; 0.9 us through ctypes
+def _workspace_bytes(*sizes):
+    return int(_lib.load().coopt_verify_attention_workspace(*sizes))
+
+
 def workspace_bytes(batch: int, num_heads: int, num_kv_heads: int, head_dim: int,
                     max_seqlen_q: int, max_seqlen_k: int) -> int:
-    return int(_lib.load().coopt_verify_attention_workspace(batch, num_heads, num_kv_heads,
-                                                            head_dim, max_seqlen_q, max_seqlen_k))
+    """Bytes paged_attention needs; sizes as integers or anything with an integer value (NumPy
+    scalars and 0-d arrays, one-element tensors)."""
+    return _workspace_bytes(*map(operator.index, (batch, num_heads, num_kv_heads, head_dim,
+                                                  max_seqlen_q, max_seqlen_k)))
 
 
 def paged_attention(q, k_cache, v_cache, cu_seqlens_q, seq_lens, block_table, max_seqlen_q,
@@ -82,7 +89,7 @@ def paged_attention(q, k_cache, v_cache, cu_seqlens_q, seq_lens, block_table, ma
     cu = cu_seqlens_q.contiguous()
     sl = seq_lens.contiguous()
     lib = _lib.load()
-    need = workspace_bytes(B, Hq, Hkv, D, int(max_seqlen_q), int(max_seqlen_k))
+    need = _workspace_bytes(B, Hq, Hkv, D, int(max_seqlen_q), int(max_seqlen_k))
     if workspace is None:
         workspace = _WS.get(need, q.device)
     elif workspace.numel() * workspace.element_size() < need:
@@ -178,7 +185,7 @@ def paged_attention_qkv(qkv, positions, cos, sin, slot_mapping, k_cache, v_cache
         raise ValueError("out must be bf16 [T, Hq, D] with contiguous D")
     if B == 0 or T == 0:
         return out
-    need = workspace_bytes(B, Hq, Hkv, D, int(max_seqlen_q), int(max_seqlen_k))
+    need = _workspace_bytes(B, Hq, Hkv, D, int(max_seqlen_q), int(max_seqlen_k))
     if workspace is None:
         workspace = _WS.get(need, dev)
     elif workspace.numel() * workspace.element_size() < need:

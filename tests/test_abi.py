@@ -5,6 +5,7 @@ import ctypes
 import os
 import re
 
+import numpy as np
 import pytest
 import torch  # noqa: F401  (must precede the library load)
 
@@ -53,6 +54,25 @@ def test_workspace_sizes_are_positive_and_monotone(lib):
     c = lib.coopt_accept_sample_workspace(8, 4, 128256)
     d = lib.coopt_accept_sample_workspace(32, 4, 128256)
     assert 0 < c < d
+
+
+def test_workspace_bytes_follow_the_sizes_values(lib):
+    """Sizes given as 0-d arrays and tensors count by their value at the call, also when the same
+    object holds another one later; what has no integer value is refused."""
+    from iitj_llm_coopt_amd.attention import workspace_bytes
+
+    small, large = workspace_bytes(2, 32, 8, 128, 5, 600), workspace_bytes(2, 32, 8, 128, 5, 6000)
+    assert 0 < small < large
+    keys = torch.tensor(600)
+    assert workspace_bytes(2, 32, 8, 128, 5, keys) == small
+    keys.fill_(6000)
+    assert workspace_bytes(2, 32, 8, 128, 5, keys) == large
+    assert workspace_bytes(2, 32, 8, 128, np.array(5), np.int64(6000)) == large
+    assert workspace_bytes(batch=2, num_heads=32, num_kv_heads=8, head_dim=128, max_seqlen_q=5,
+                           max_seqlen_k=600) == small
+    for bad in (600.0, "600", None):
+        with pytest.raises(TypeError):
+            workspace_bytes(2, 32, 8, 128, 5, bad)
 
 
 def _err(rc):
