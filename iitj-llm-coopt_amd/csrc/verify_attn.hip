@@ -1155,8 +1155,9 @@ __global__ __launch_bounds__(kThreads) void merge_kernel(AttnArgs a) {
 // probabilities with ones: 67.4 us, and no longer a sum of 32-bit probabilities.)
 // Tried: 64 keys per softmax (66-72 us, but 50 instead of 42 us for 2000 keys of a verify item alone,
 // which two waves share below), one stage of loads in flight with an L2 touch ahead (72).
-// Blocks take the windows with most keys first: window r from the end of every sequence before
-// window r + 1 of any (B <= kPlanSeqs; larger batches run in grid order).
+// Blocks take every sequence's last window first, then every one's last but one, and so on
+// (B <= kPlanSeqs; larger batches run in grid order): a chunk's windows with most keys ahead of its
+// others, and no block without rows among them. Sequences are not ranked by their keys.
 constexpr int kPrefillRows = 128;
 constexpr int kStageKeys = 64;
 

@@ -449,12 +449,13 @@ def test_windowed_call_needs_no_partials_workspace(dev):
 @pytest.mark.parametrize("ctx,q_lens", [
     ([0, 14, 15, 30, 31, 63, 254, 700], [1] * 8),     # last tiles of 1 to 32 keys, 1 to 3 splits
     ([15, 250, 1999], [5, 1, 5]),                     # 8 splits
-    ([16001], [5]),                                   # 63 splits: eight merge rounds
+    ([10000], [5]),                                   # 20: merged 8 + 8 + 4 (D 64: 16 + 4)
+    ([16001], [5]),                                   # 32: whole merge rounds
     ([3, 200], [33, 20]),                             # query windows
 ])
 def test_rows_past_the_end_and_many_splits(dev, kv, D, ctx, q_lens):
-    """Cache rows past a sequence's end hold NaN (INT8: infinite scales) here; the tile loads
-    that cover them must not let them reach a result.  Tolerances as at the top."""
+    """Cache rows past a sequence's end hold NaN (INT8: infinite scales) here; none may reach a
+    result.  Tolerances as at the top."""
     pool = Pool(ctx, q_lens, 32, 8, D, dev, kv=kv, seed=len(ctx) + D, slack=5)
     written = torch.zeros(pool.kc.shape[:2], dtype=torch.bool, device=dev)
     for b in range(len(ctx)):
@@ -509,3 +510,59 @@ def test_long_chunks_match_the_oracle(dev, long_windows, kv, D, G, ctx, q_lens, 
     excess, mx, ulps = pool.max_err(out, sorted(set(seqs)))
     report(f"[long chunks {kv} D={D} G={G}] excess {excess:.4f} max-abs {mx:.4f} ulps {ulps:.2f}")
     assert excess <= (TOL_BF16 if kv == "auto" else TOL_INT8)
+
+
+@pytest.mark.parametrize("kv", ["auto", "int8"])
+@pytest.mark.parametrize("D,G", [(128, 3), (64, 7), (128, 64)])
+def test_long_chunks_in_other_layouts(dev, long_windows, kv, D, G):
+    """The prefill kernel over token-major caches and scales, over one layer of a block-major
+    buffer, and with q and out as strided views: bit for bit what it gives over head-major caches and
+    contiguous rows.  G does not divide the 128 rows of a window; the second sequence has fewer
+    keys than rows (its first rows see none and are zero)."""
+    Hkv, ctx, q_lens = 2, [300, 0, 40], [90, 70, 3]
+    long_windows(kv, Hkv * G, Hkv, D, ctx, q_lens)
+    pool = Pool(ctx, q_lens, Hkv * G, Hkv, D, dev, kv=kv, seed=D + G, slack=2)
+    full = pool.run()
+    excess, mx, ulps = pool.max_err(full)
+    report(f"[long chunks {kv} D={D} G={G}] excess {excess:.4f} max-abs {mx:.4f} ulps {ulps:.2f}")
+    assert excess <= (TOL_BF16 if kv == "auto" else TOL_INT8)
+
+    pool.seq_lens[1] -= 37
+    want = pool.run()
+    assert (want[90:127] == 0).all() and torch.equal(want[:90], full[:90])
+    head_major = (pool.kc, pool.vc, pool.ks, pool.vs)
+
+    def as_layer(t):       # layer 1 of [blocks, layers, ...]
+        buf = torch.zeros((t.shape[0], 3) + tuple(t.shape[1:]), dtype=t.dtype, device=dev)
+        buf[:, 1] = t
+        return buf[:, 1]
+
+    for relaid in (lambda t: t.contiguous(), as_layer):
+        pool.kc, pool.vc, pool.ks, pool.vs = (None if t is None else relaid(t) for t in head_major)
+        assert torch.equal(pool.run(), want)
+        T, Hq = pool.q.shape[:2]
+        qbuf = torch.zeros(T, 2, Hq, D + 8, dtype=torch.bfloat16, device=dev)
+        qbuf[:, 1, :, :D] = pool.q
+        obuf = torch.full((T, Hq, D + 16), 7.0, dtype=torch.bfloat16, device=dev)
+        pool.run(q=qbuf[:, 1, :, :D], out=obuf[..., :D])
+        assert torch.equal(obuf[..., :D], want) and (obuf[..., D:] == 7).all()
+
+
+def test_long_chunks_int8_v_scales_move_the_reference(dev, long_windows):
+    """V magnitudes log-uniform over [1e-3, 1e6] per (token, head) move the prefill kernel's V-scale
+    reference in the middle of a window, by waves alone and by pairs of waves.  The bar of the
+    short items' test above: 2e-2 of the sequence's largest output."""
+    ctx, q_lens = [37, 700, 64], [100, 40, 5]
+    rng = np.random.default_rng(3)
+    mag = (10.0 ** rng.uniform(-3, 6, (sum(ctx) + sum(q_lens), 8))).astype(np.float32)
+    long_windows("int8", 32, 8, 128, ctx, q_lens)
+    pool = Pool(ctx, q_lens, 32, 8, 128, dev, "int8", seed=21, vmag=mag)
+    out = pool.run()
+    assert torch.isfinite(out.float()).all()
+    o = out.float().cpu().numpy()
+    for b in range(len(ctx)):
+        q0, q1 = int(pool.cu[b]), int(pool.cu[b + 1])
+        ref = pool.oracle_seq(b)
+        rel = float(np.abs(o[q0:q1] - ref).max() / np.abs(ref).max())
+        report(f"[long chunks V scales, sequence {b}] relative to its largest output {rel:.3g}")
+        assert rel <= 2e-2
