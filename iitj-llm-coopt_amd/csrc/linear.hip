@@ -15,7 +15,7 @@
 //     contiguous bytes of its output row as 4 x 16 B (MFMA j covers k0 + 32j + [8g, 8g+8),
 //     g = lane / 16), PF steps ahead of the MFMAs.
 //   * X is shared: each K step's [M, 128] slice is staged once per workgroup in LDS (double
-//     buffered, rows padded to 288 bytes) and read by all waves as MFMA A operands.
+//     buffered, rows padded to 272 or 288 bytes: pitch_for) and read by all waves as MFMA A operands.
 //   * v_mfma_f32_16x16x32_bf16 with A = X rows, B = W rows: lane l holds
 //     C[4(l/16) + i][l % 16] of each 16x16 tile (SILU: A = W, B = X, the transpose).
 //
@@ -42,9 +42,10 @@ constexpr int kKB = 128;                  // K elements per step
 // LDS bytes per staged X row.  A fragment read has 16 lanes at consecutive rows and four 16-byte
 // columns; at a pitch of 288 it takes 4.1 cycles per 1 KB, the rate of a contiguous read, at 272
 // (one 16-byte unit of padding) 7.0: bank conflicts on 41 of the 93 kcycles the LDS was busy in
-// a 160 x 28672 x 4096 call.  160 rows, partials: gate_up 64 -> 57 us, down 35.1 -> 31.9, qkv
-// 24.6 -> 23.0.
-constexpr int kPitch = kKB * 2 + 32;
+// a 160 x 28672 x 4096 call.  160 rows, partials, 272 / 288: down 36.2 / 32.0 us, qkv 21.1 / 18.5.
+// Row-major weights of up to 64 rows are 1 to 3 % faster at 272 (their loads, not the LDS, take the time:
+// 64 x 6144 x 4096 16.4 / 16.8 us).
+constexpr int pitch_for(bool pk, int mt) { return kKB * 2 + (pk || mt > 4 ? 32 : 16); }
 
 struct LinArgs {
   const uint16_t* x;
@@ -98,6 +99,7 @@ __global__ __launch_bounds__(64 * WAVES) void linear_kernel(
   constexpr int kThreads = 64 * WAVES;
   constexpr int kRowsPerRound = kThreads / 16;                     // X rows staged per round
   constexpr int kRounds = (MT * 16 + kRowsPerRound - 1) / kRowsPerRound;
+  constexpr int kPitch = pitch_for(PK, MT);
   // whole rounds: with a row count that they do not divide, the rows past it have LDS of their
   // own, and packed weights' stores (store_x) need no branch
   __shared__ __attribute__((aligned(16))) unsigned char xs[2][kRounds * kRowsPerRound * kPitch];
@@ -373,7 +375,7 @@ Plan plan_for(int M, int N, int K) {
   };
   int ks = split_for(p.waves);
   // 160 rows: 7 waves (112 columns) where that fills more of the 256 CUs than 8 do -- the
-  // target's qkv, N = 6144: 55 x 4 = 220 workgroups against 48 x 4 = 192, 22.2 -> 20.5 us
+  // target's qkv, N = 6144: 55 x 4 = 220 workgroups against 48 x 4 = 192, 19.1 -> 18.5 us
   if (p.mt == 10 && p.nw == 1 && p.waves == 8) {
     const int k7 = split_for(7);
     if (((N + 111) / 112) * k7 > ((N + 127) / 128) * ks && ((N + 111) / 112) * k7 <= 256) {
