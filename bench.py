@@ -282,6 +282,32 @@ def attention_case(torch, M, dev, ctx, qlen, kv_dtype, seed, D=128, cpu_sample=0
     return res
 
 
+def mixed_prefill_case(torch, M, dev, seed, Hq=32, D=128):
+    """Prefill chunks of 1500 and 500 tokens (the second over 1000 cached ones) and 16 verify items of
+    5 tokens over 300 to 2100 in one call, bf16: prefill_attn_kernel.  The flops are those of the
+    visible (row, key) pairs."""
+    import numpy as np
+
+    n = np.array([1500, 500] + [5] * 16)
+    keys = n + np.concatenate([[0, 1000], np.random.default_rng(seed).integers(300, 2101, 16)])
+    st = attention_setup(torch, M, dev, keys.tolist(), 0, "auto", seed, D, 0.0, "head")
+    kc, vc, ks, vs = st["caches"]
+    cu = torch.from_numpy(np.concatenate([[0], np.cumsum(n)]).astype(np.int32)).to(dev)
+    T = int(n.sum())
+    q = torch.randn(T, Hq, D, generator=st["gen"], device=dev).to(torch.bfloat16)
+    out = torch.empty_like(q)
+
+    def fn():
+        M.paged_attention(q, kc, vc, cu, st["sl"], st["table"], 1500, int(keys.max()), D ** -0.5,
+                          ks, vs, out)
+
+    pairs = int((n * (keys - n) + n * (n + 1) // 2).sum())
+    res = rate({"kv": "auto", "head_dim": D, "batch": len(n), "q_tokens": T, "flops": 4 * D * Hq * pairs},
+               int(keys.sum()) * st["per_tok"] + 2 * T * Hq * D * 2, *time_launches(torch, dev, fn))
+    res["TFLOP_s"] = res["flops"] / (res["avg_us"] * 1e-6) / 1e12
+    return res
+
+
 def attention_qkv_case(torch, M, dev, ctx, qlen, kv_dtype, seed, D=128, hidden=4096):
     """The step's form of the call: coopt_verify_attention_qkv, the qkv projection's split-K
     partials in (coopt_linear_packed with defer_reduce, as the step runs it: hidden -> (Hq +
@@ -649,6 +675,23 @@ def linear_case(torch, M, dev, rows, n, k, seed, packed=False):
     return res
 
 
+def linear_silu_case(torch, M, dev, rows, f, k, seed):
+    """gate_up with SiLU and the product fused (fused.linear_silu, coopt_linear_silu_packed), bf16,
+    N(0,1) x, N(0, 0.02^2) weights.  Algorithmic bytes: the weight, x and the output once each."""
+    g = torch.Generator(device=dev).manual_seed(seed)
+    x = torch.randn(rows, k, generator=g, device=dev).to(torch.bfloat16)
+    w = M.fused.pack_gate_up_weight((torch.randn(2 * f, k, generator=g, device=dev) * 0.02).to(torch.bfloat16))
+    y = torch.empty(rows, f, dtype=torch.bfloat16, device=dev)
+
+    def fn():
+        M.fused.linear_silu(x, w, out=y)
+
+    res = rate({"rows": rows, "f": f, "k": k, "flops": 4 * rows * f * k},
+               2 * f * k * 2 + rows * k * 2 + rows * f * 2, *time_launches(torch, dev, fn))
+    res["TFLOP_s"] = res["flops"] / (res["avg_us"] * 1e-6) / 1e12
+    return res
+
+
 def copy_case(torch, M, dev, seed):
     """A plain streaming kernel of known size (torch.neg over 1 GiB of bf16: 1 GiB read,
     1 GiB written): the calibration for FETCH_SIZE / WRITE_SIZE and a practical HBM ceiling."""
@@ -693,6 +736,8 @@ KERNEL_CASES = {
     # the same launches as the step makes them: the qkv epilogue inside the attention launch
     "attention_qkv_step_target": lambda t, M, d, s: attention_qkv_case(t, M, d, [1100] * 32, 5, "int8", s),
     "attention_qkv_step_draft": lambda t, M, d, s: attention_qkv_case(t, M, d, [1100] * 32, 1, "auto", s, D=64, hidden=2048),
+    # prefill chunks and verify items in one call
+    "attention_mixed_prefill": lambda t, M, d, s: mixed_prefill_case(t, M, d, s),
     # config 1 (B=8) and the metric's B=32
     "accept_b8": lambda t, M, d, s: accept_case(t, M, d, 8, 4, 128256, s),
     "accept_b32": lambda t, M, d, s: accept_case(t, M, d, 32, 4, 128256, s),
@@ -708,9 +753,10 @@ KERNEL_CASES = {
     "codec_quantize_64MiB": lambda t, M, d, s: codec_case(t, M, d, s, "quantize"),
     "codec_dequantize_64MiB": lambda t, M, d, s: codec_case(t, M, d, s, "dequantize"),
     "kv_migrate_256x2MiB": lambda t, M, d, s: migrate_case(t, M, d, s),
-    # the step's weight-streaming projections, tile-packed as in the step: target qkv / down
+    # the step's weight-streaming projections, tile-packed as in the step: target qkv / gate_up / down
     # at the verify rows (B (gamma+1) = 160), draft lm_head at the draft rows (B = 32)
     "linear_m160_qkv": lambda t, M, d, s: linear_case(t, M, d, 160, 6144, 4096, s, packed=True),
+    "linear_m160_gate_up_silu": lambda t, M, d, s: linear_silu_case(t, M, d, 160, 14336, 4096, s),
     "linear_m160_down": lambda t, M, d, s: linear_case(t, M, d, 160, 4096, 14336, s, packed=True),
     "linear_m32_lm_head": lambda t, M, d, s: linear_case(t, M, d, 32, 128256, 2048, s, packed=True),
     "copy": lambda t, M, d, s: copy_case(t, M, d, s),
