@@ -40,9 +40,8 @@ typedef uint32_t u32x2_any_t __attribute__((ext_vector_type(2), aligned(2)));
 
 constexpr int kKB = 128;                  // K elements per step
 // LDS bytes per staged X row.  A fragment read has 16 lanes at consecutive rows and four 16-byte
-// columns; at a pitch of 288 it takes 4.1 cycles per 1 KB, the rate of a contiguous read, at 272
-// (one 16-byte unit of padding) 7.0: bank conflicts on 41 of the 93 kcycles the LDS was busy in
-// a 160 x 28672 x 4096 call.  160 rows, partials, 272 / 288: down 36.2 / 32.0 us, qkv 21.1 / 18.5.
+// columns: at a pitch of 288 no bank conflicts, at 272 (one 16-byte unit of padding) 4.6 of the 10.4 M
+// cycles that the LDS is busy in a 160 x 4096 x 14336 call, 5.8 M at 288.  160 rows, partials, 272 / 288: down 36.2 / 32.0 us, qkv 21.1 / 18.5.
 // Row-major weights of up to 64 rows are 1 to 3 % faster at 272 (their loads, not the LDS, take the time:
 // 64 x 6144 x 4096 16.4 / 16.8 us).
 constexpr int pitch_for(bool pk, int mt) { return kKB * 2 + (pk || mt > 4 ? 32 : 16); }

@@ -19,7 +19,7 @@
 // Items of more than 64 rows (prefill chunks of a mixed batch) are cut into query windows -- each
 // window is itself a sequence of those rows over the keys its last row sees -- and run one
 // unsplit block per (window, KV head): windows of 64/G query tokens here, of 128/G in
-// prefill_attn_kernel, which takes the calls with long chunks.
+// prefill_attn_kernel, which takes the calls whose windows fill the GPU (prefill_is_faster).
 //
 // MFMA layout (v_mfma_f32_16x16x32_{bf16,f16}; lane l, g = l/16, m = l%16):
 //   scores  S^T[key][row] = sum_d K[key][d] Q[row][d]     A = K, B = Q^T
@@ -54,8 +54,6 @@
 // 8.3e6): it is set from the largest V scale seen so far and enters the softmax exponent, so
 // it cancels in o / l like the running max does.
 #include <math.h>
-
-#include <type_traits>
 
 #include "common.h"
 #include "kv_store.h"
@@ -1147,9 +1145,9 @@ __global__ __launch_bounds__(kThreads) void merge_kernel(AttnArgs a) {
 // selects as build_va does, with two stages of global loads in flight.  Operands, softmax and
 // number formats are verify_attn_kernel's; Q lives in registers.  64 KB of LDS and 256 registers
 // let two blocks share a CU.
-// What bounds it: a wave's own instruction stream (about 165 VALU and 32 MFMA instructions a tile
-// and 32 rows) and, where windows are few, its chain per stage (1.3-2 us: staging 1.0 without the
-// tiles' work, the tiles 0.5-1.0).  Chunks of 1500 and 500 rows with 16 verify items of 5 rows
+// What bounds it: a wave's own instruction stream (by the listing about 165 VALU and 32 MFMA instructions
+// a tile and 32 rows; counted over the batch below, staging included, 7.3 VALU per MFMA) and, where windows are few, its chain per stage (1.3-2 us: staging 1.0 without the
+// tiles' work, the tiles 0.5-1.0).  Chunks of 1500 and 500 tokens with 16 verify items of 5
 // (bf16, 32/8 heads of 128, 30 GFLOP): 138 us on verify_attn_kernel's windows of 64 rows, whose
 // waves each read their own keys, 66 us here; INT8 190 and 82.  (l as a product of the rounded
 // probabilities with ones: 67.4 us, and no longer a sum of 32-bit probabilities.)
@@ -1599,7 +1597,7 @@ __global__ __launch_bounds__(256, 2) void prefill_attn_kernel(AttnArgs a) {
 // than one split is split, so shorter ones run whole.  Contexts of up to kWholeRounds rounds
 // are not split however few the items are (1 sequence, 8 KV heads, bf16, 1 row, 400 keys: 9.0 us
 // whole, the merge launch alone costs 3); past that a split may be as short as one round (717
-// keys: 11.3 us whole, 11.9 in splits of two rounds, 9.7 of one; 4096 keys: 14.1 and 12.6).
+// keys: 11.6 us whole, 11.8 in splits of two rounds, 9.8 of one; 4096 keys: 13.2 and 11.7).
 constexpr int kWholeRounds = 2;
 int target_blocks(int waves) { return waves == 8 ? 256 : 512; }
 

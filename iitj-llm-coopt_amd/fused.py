@@ -224,7 +224,8 @@ def linear(x, weight, out=None, defer_reduce=False):
     up to LINEAR_MAX_ROWS rows, and runs where it measured faster than torch's GEMM on MI355X:
     up to 64 rows (draft steps), or N <= 8192 outputs at any supported row count (the verify
     step's qkv / o / down projections).  Other shapes -- prefill-sized row counts, and the
-    wide gate_up / lm_head outputs at verify row counts -- go to torch (hipBLASLt).
+    wide gate_up / lm_head outputs at verify row counts -- go to torch (hipBLASLt); linear_silu
+    has a fused kernel for a packed gate_up at verify row counts.
 
     defer_reduce=True (no `out`): on the kernel path, return a LinearPartials instead of the
     tensor, for rms_norm() or silu_and_mul() to reduce in their own pass; other paths return

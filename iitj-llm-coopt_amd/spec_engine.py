@@ -102,8 +102,9 @@ class RandomLlama:
         self.scale = 1.0 / math.sqrt(D)
 
     # Projections kept tile-packed as well on the GPU: those that stream through coopt_linear
-    # at verify row counts, gate_up with its SiLU fused (160 rows of the 8B widths: 54 us against
-    # 57 + 6 us of torch's GEMM and silu_and_mul).  A model run only at draft row counts (<= 64)
+    # at verify row counts, gate_up with its SiLU fused (160 rows of the 8B widths: 51 to 54 us
+    # against 65 us of torch's GEMM and silu_and_mul).  The second copy of gate_up is read at up
+    # to 64 and at 129 to 160 rows; other row counts use torch's GEMM.  A model run only at draft row counts (<= 64)
     # streams its logits projection through it too, and passes
     # packed=("qkv", "o", "gate_up", "down", "lm_head").  At 160 rows the target's lm_head
     # runs on torch's GEMM (245 us; coopt_linear_packed 242).
@@ -159,7 +160,7 @@ class RandomLlama:
             if attn is None:
                 q = ops.qkv_epilogue(kv, li, qkv, pos, self.cos, self.sin, slots, H, Hkv, D)
                 attn = ops.attend(kv, li, q, meta, self.scale)
-            # gate_up + SiLU·mul is one launch at draft row counts (linear_silu); o, down and
+            # gate_up + SiLU·mul is one launch at draft and verify row counts (linear_silu); o, down and
             # otherwise gate_up feed only the fused add + norm or SiLU, which reduce their
             # split-K partials as they read them
             o = ops.linear(attn.reshape(T, H * D), L["o"], defer_reduce=True)
