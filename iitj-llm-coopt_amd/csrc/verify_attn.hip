@@ -70,7 +70,7 @@ constexpr int kThreads = 256;  // merge kernel
 // Waves per attention block: 8 (one block per CU at two waves per SIMD, i.e. at most 256
 // registers per lane) while the accumulators and two tile buffers fit that (RT <= 3), else 4.
 constexpr int waves_for(int RT) { return RT <= 3 ? 8 : 4; }
-// Blocks that share a CU: two with 4 waves at head dim 64 and bf16 (76 KB of LDS, at most 256 registers
+// Blocks that share a CU: two with 4 waves at head dim 64 and bf16 (79 KB of LDS, at most 256 registers
 // asked for), where batches of many query windows take 0.63 to 0.8 of the time; see alone_lds.
 constexpr int blocks_per_cu(int D, bool int8, int RT) { return D == 64 && !int8 && RT == 4 ? 2 : 1; }
 constexpr int kTileKeys = 32;
@@ -1731,7 +1731,7 @@ constexpr bool fused_ok(int D, bool int8, int RT) {
   return RT >= 1 && RT <= kFusedMaxRT && (int8 || D != 128 || RT == 1);
 }
 
-// LDS asked for beside a 64-row block's own (76 KB at head dim 64, bf16), so that no second one fits its
+// LDS asked for beside a 64-row block's own (79 KB at head dim 64, bf16), so that no second one fits its
 // CU.  Two a CU raise the rate (batches of more than 256 windows: 0.73 of the time), but windows that a
 // block on each CU would hold then double up on some of them: 5 sequences with one chunk of 286 tokens
 // over 1500 keys, 176 windows among 720 blocks, 25.4 us with two a CU and 21.7 with one.  360 batches,
